@@ -29,7 +29,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, HERE)
 
 FP32_PEAK_TFLOPS = 157.3
-# HBM bytes per launch of mcmc_kernel<3,18,false> on the full 250,968-voxel
+# HBM bytes per launch of mcmc_kernel<3,18,2,false,false> on the full 250,968-voxel
 # workload: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE, each scaled by the same
 # counter's reading for a copy kernel of known size (profiles/mcmc_c1_traffic.md)
 MCMC_TRAFFIC_BYTES = (2 * 148124 + 632652) * 1024
@@ -753,7 +753,7 @@ def main():
                    "mcmc_tile": f"{tm['lanes']} lanes x {tm['vpl']} volumes per voxel"},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP32_PEAK_TFLOPS, "traffic": traffic,
-                     "kernel": "mcmc_kernel<3,18,false,false>", "flops_per_launch": fl_launch,
+                     "kernel": "mcmc_kernel<3,18,2,false,false>", "flops_per_launch": fl_launch,
                      "compute": "FP32 vector ALU (no matrix-shaped work on this path); peak is the published "
                                 "FP32 figure, which counts packed FP32 -- this build disables packed FP32, so "
                                 "half of it (78.6) is the reachable issue ceiling"},

@@ -8,12 +8,19 @@
 // nburn + njumps sweeps.  Layout: one voxel per 16-lane DPP row, four voxels
 // per wave64.  Lane l of a row holds volumes l, l+16, l+32, ... (VPL volumes
 // per lane) and keeps, in VGPRs,
-//   the residual r = y - S0*M (Gaussian) or the data y (Rician),
+//   the residual r = y - S0*M (Gaussian) or the terms of the volumes (Rician),
 //   the mixture M = sum_k f_k s_k + (1 - f0 - sum_k f_k) iso + f0,
 //   the isotropic signal iso and the stick signals s_k;
-// The candidate stick signals of the diffusivity proposals are parked in LDS
-// (one block per wave, lane-interleaved) so that an accepted move copies them;
-// K=3 at 18 volumes per lane fits two waves per SIMD.
+// one of these arrays and the arguments b (g.x_k)^2 of the stick signals live
+// in LDS (one block per wave, lane-interleaved), and K=3 at 18 volumes per
+// lane fits two waves per SIMD.
+// The kernel is bound by VALU issue (99% of the SIMD cycles before, on the
+// 250,968-voxel multi-shell volume at K=3), so what counts is instructions per
+// sweep: evaluating what belongs to a slot once per sweep in its own lane,
+// keeping the stick arguments for the diffusivity moves and each proposal's
+// per-volume changes for its acceptance took 5,107 VALU instructions per wave
+// and sweep to 4,193, and one kernel per model (128 KB of code to 54, no
+// spilled vector registers) let the launch follow: 1,247 to 1,020 ms.
 // A proposal evaluates only what it changes; its likelihood change is
 // summed over the row with DPP adds.  For Gaussian noise a move of every
 // residual by -c*q gives the change of the sum of squares c*(c*sum q^2 -
@@ -85,32 +92,32 @@ template <int VPL> constexpr bool ZERO_SLOT = VPL == 18;
 // factor leaves an exponent error below d u 2^-24 for every w (e <= half an
 // ulp of u1, and (d^2/dstd^2) w = d u).
 struct SigC {
-  int kind;
   float c0, c1;
 };
+// the stick and isotropic forms of a model (model 3: zeppelins with the
+// gamma-distributed isotropic term)
+template <int MODEL> constexpr int STICK_KIND = MODEL - 1;
+template <int MODEL> constexpr int ISO_KIND = MODEL == 1 ? 0 : 1;
 FDT_DEV SigC gamma_coef(float d, float dstd) {
   SigC c;
-  c.kind = 1;
   if (dstd < 1e-5f) { c.c0 = 0x1p-64f; c.c1 = -d * 0x1p64f; }
   else { const float s2 = dstd * dstd; c.c0 = s2 / d; c.c1 = -(d * d / s2); }
   return c;
 }
-FDT_DEV SigC aniso_coef(int model, float d, float dstd, float R) {
-  SigC c;
-  if (model == 1) { c.kind = 0; c.c0 = -d * L2E; c.c1 = 0.0f; }
-  else if (model == 2) c = gamma_coef(d, dstd);
+template <int MODEL>
+FDT_DEV SigC aniso_coef(float d, float dstd, float R) {
+  if constexpr (MODEL == 1) return SigC{-d * L2E, 0.0f};
+  else if constexpr (MODEL == 2) return gamma_coef(d, dstd);
   else {
     float iR = 1.0f / (2.0f * R + 1.0f);
     float k = -3.0f * d * iR * L2E;
-    c.kind = 2; c.c0 = k * (1.0f - R); c.c1 = k * R;
+    return SigC{k * (1.0f - R), k * R};
   }
-  return c;
 }
-FDT_DEV SigC iso_coef(int model, float d, float dstd) {
-  SigC c;
-  if (model == 1) { c.kind = 0; c.c0 = -d * L2E; c.c1 = 0.0f; }
-  else c = gamma_coef(d, dstd);
-  return c;
+template <int MODEL>
+FDT_DEV SigC iso_coef(float d, float dstd) {
+  if constexpr (MODEL == 1) return SigC{-d * L2E, 0.0f};
+  else return gamma_coef(d, dstd);
 }
 template <int SK>
 FDT_DEV float sig(const SigC& c, float u, float b) {
@@ -122,13 +129,6 @@ FDT_DEV float sig(const SigC& c, float u, float b) {
   }
   else return ex2(fmaf(c.c0, u, c.c1 * b));
 }
-template <class F>
-FDT_DEV void by_kind(int kind, F&& f) {
-  if (kind == 0) f(std::integral_constant<int, 0>{});
-  else if (kind == 1) f(std::integral_constant<int, 1>{});
-  else f(std::integral_constant<int, 2>{});
-}
-
 // log I0 by Abramowitz-Stegun 9.8.1/9.8.2 (fibre.h:29-48, CUDA/runmcmc_kernels.cu:126-145)
 FDT_DEV float logI0f(float x) {
   float b = fabsf(x);
@@ -141,6 +141,13 @@ FDT_DEV float logI0f(float x) {
   // one logarithm of the selected branch: log ys, or b + log(pl / sqrt b)
   const bool sm = b < 3.75f;
   return flog(sm ? ys : pl * __builtin_amdgcn_rsqf(b)) + (sm ? 0.0f : b);
+}
+// log I0 above 3.75 alone, the same operations
+FDT_DEV float logI0_large(float x) {
+  const float b = fabsf(x);
+  float c = 3.75f * __builtin_amdgcn_rcpf(b);
+  float pl = 0.39894228f + c * (0.01328592f + c * (0.00225319f + c * (-0.00157565f + c * (0.00916281f + c * (-0.02057706f + c * (0.02635537f + c * (-0.01647633f + c * 0.00392377f)))))));
+  return flog(pl * __builtin_amdgcn_rsqf(b)) + b;
 }
 // Rician log-likelihood term of one volume (fibre.h:949-953),
 //   log y - tau (y^2 + p^2) / 2 + log I0(tau p y),
@@ -184,7 +191,7 @@ FDT_DEV int rej1(int c) { return c + (1 << 16); }
 // the stick signals use the shared acquisition with the fibre directions
 // mapped by M^T, and the isotropic signal (and the model-3 R term) the
 // voxel's own b values, kept per row in LDS.
-template <int K, int VPL, bool RIC, bool GN = false>
+template <int K, int VPL, int MODEL, bool RIC, bool GN = false>
 struct Chain {
   // lane-resident volume state, volume i = rl + 16 t.  One per-volume
   // array lives in the wave's LDS block `vol` instead of registers (18
@@ -198,7 +205,14 @@ struct Chain {
   float iso_r[ISO_LDS ? 1 : VPL];
   float s[K][VPL];
   float* vol;   // wave's LDS block: vol[t*64]
-  float* cand;  // candidate stick signals of the diffusivity proposals, wave's LDS block: cand[(k*VPL+t)*64]
+  // The wave's LDS block sk[(k*VPL+t)*64] holds the arguments b (g.x_k)^2 of
+  // the stick signals (U_LDS): the diffusivity proposals read them there and
+  // keep their candidate signals in registers.  Where the registers do not
+  // allow that, it holds the candidate signals, and the arguments are formed
+  // from the fibre directions again.
+  static constexpr int HELD = VPL * (2 * K + 3 + !ISO_LDS + RIC);  // floats a lane holds in a diffusivity proposal
+  static constexpr bool U_LDS = HELD <= (RIC ? 130 : 162) * (VPL > 18 ? 2 : 1);
+  float* sk;
   float ell[RIC ? VPL : 1];
   // isotropic signal per b-shell (acquisitions with <= 16 distinct b values):
   // sh[i] is the shell of volume i, shb[l] its b value, isot the row's table
@@ -208,12 +222,18 @@ struct Chain {
   int nshell;
   float sval, sprop, sprior;
   int scnt;
-  // sin and cos of the slot's angle (theta_k / phi_k slots), kept with the
-  // value so that fibre directions are row broadcasts, not re-evaluated.
-  // The d slot holds the stick-signal coefficients of the current state
-  // there instead (c0, c1), set whenever d, d_std or R moves, so that the
-  // angle proposals broadcast them instead of dividing again.
+  // sin and cos of the slot's angle (theta_k / phi_k slots), kept with the value
   float ssin, scos;
+  // The slots' candidates of the current sweep (propose): a slot's value and
+  // width change only with its own proposal, so every candidate, its sine and
+  // cosine and its prior are known when the sweep begins and each lane
+  // evaluates its own slot's once, instead of the whole row at every proposal.
+  float sxn, ssn, scn, sprn, sdp;
+  uint32_t accm;  // slots accepted in the current sweep (bit: slot), settled at its end
+  int rejinc;     // what a rejection adds to the slot's counters (0: not sampled)
+  // row-uniform copies of the parameters that other slots' proposals read
+  float S0, tau, d, dstd, Rr, f0, fk[K], fsum;
+  SigC ca;        // stick-signal coefficients of the current state
   double like;  // Gaussian: SSR; Rician: sum of ell
   int nv;       // slots of this lane that hold a real volume (rl + 16 t < N)
   int rl;
@@ -222,7 +242,6 @@ struct Chain {
   bool z0;
   FDT_DEV bool skip(int t) const { return ZERO_SLOT<VPL> && t == 0 && z0; }
   // options
-  int model;
   bool incf0, ardf0, can_ard;
   bool lam[K];
   float fudge, halfN, Nf, Rmean, Rstd, Rfudge;
@@ -248,15 +267,11 @@ struct Chain {
   static constexpr int TH(int k) { return SL_FIB + 3 * k; }
   static constexpr int PH(int k) { return SL_FIB + 3 * k + 1; }
   static constexpr int FK(int k) { return SL_FIB + 3 * k + 2; }
-  template <int SL> FDT_DEV float v() const { return row_bcast<SL>(sval); }
-  template <int SL> FDT_DEV float width() const { return row_bcast<SL>(sprop); }
-  template <int SL> FDT_DEV float prior() const { return row_bcast<SL>(sprior); }
-  template <int SL> FDT_DEV void reject() { if (rl == SL) scnt += 1 << 16; }
-  template <int SL> FDT_DEV void accept(float val, float prn) {
-    if (rl == SL) { sval = val; scnt += 1; sprior = prn; }
-  }
+  template <int SL> FDT_DEV float cand() const { return row_bcast<SL>(sxn); }    // the slot's candidate
+  template <int SL> FDT_DEV float dprior() const { return row_bcast<SL>(sdp); }  // its prior energy change
+  template <int SL> FDT_DEV void accept() { accm |= 1u << SL; }
 
-  FDT_DEV float& cnd(int k, int t) const { return cand[(k * VPL + t) * 64]; }
+  FDT_DEV float& ldsk(int k, int t) const { return sk[(k * VPL + t) * 64]; }
   FDT_DEV float& isov(int t) {
     if constexpr (ISO_LDS) return vol[t * 64];
     else return iso_r[t];
@@ -269,17 +284,6 @@ struct Chain {
   FDT_DEV float yv(int t) const {
     if constexpr (Y_LDS) return vol[t * 64];
     else return r[t];
-  }
-  // stick-signal coefficients of the current state (the kind follows the model)
-  FDT_DEV SigC aniso_cached() const {
-    SigC c;
-    c.kind = model == 1 ? 0 : (model == 2 ? 1 : 2);
-    c.c0 = row_bcast<SL_D>(ssin);
-    c.c1 = row_bcast<SL_D>(scos);
-    return c;
-  }
-  FDT_DEV void set_aniso_cache(const SigC& c) {
-    if (rl == SL_D) { ssin = c.c0; scos = c.c1; }
   }
   // unit directions of the row's fibres (from the theta / phi slots)
   struct Dirs {
@@ -305,16 +309,10 @@ struct Chain {
   // 0 there, need no mask; the S0 and diffusivity proposals, where the
   // mixture at a padding slot moves by rounding, and every Rician term do.
   FDT_DEV float mask(int t, float x) const { return t < nv ? x : 0.0f; }
-  // the fractions of the row: fk[k] and f0, their sum
-  struct Fr {
-    float fk[K];
-    float f0, sum;
-  };
-  FDT_DEV Fr fractions() const {
-    Fr q;
-    q.f0 = v<SL_F0>();
-    q.sum = q.f0;
-    sfor<K>([&](auto kc) { q.fk[kc] = v<FK(kc)>(); q.sum += q.fk[kc]; });
+  // sum of the fractions (f0 first, the order of the reference's sums)
+  FDT_DEV float sum_fractions() const {
+    float q = f0;
+    sfor<K>([&](auto kc) { q += fk[kc]; });
     return q;
   }
   // energy change of the likelihood from a row-summed change `dl`
@@ -349,21 +347,19 @@ struct Chain {
     return true;
   }
   // mixture of slot t from the stored signals
-  FDT_DEV float mix(int t, const Fr& q) const {
-    float m = fmaf(1.0f - q.sum, isov(t), q.f0);
+  FDT_DEV float mix(int t) const {
+    float m = fmaf(1.0f - fsum, isov(t), f0);
 #pragma unroll
-    for (int k = 0; k < K; ++k) m = fmaf(q.fk[k], s[k][t], m);
+    for (int k = 0; k < K; ++k) m = fmaf(fk[k], s[k][t], m);
     return m;
   }
 
   // rebuild M and the residual (or the Rician terms) from the stored signals
   FDT_DEV void rebuild(const float* y) {
-    const Fr q = fractions();
-    const float S0 = v<SL_S0>(), tau = v<SL_TAU>();
     double ss = 0.0;
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
-      float m = mix(t, q);
+      float m = mix(t);
       M[t] = m;
       if constexpr (RIC) {
         ell[t] = ell_of(yv(t), S0 * m, tau);
@@ -377,55 +373,78 @@ struct Chain {
   }
 
   // ---------------------------------------------------------- proposals
-  // n: standard normal draw, lu: log of the uniform draw of the slot.
+  // The candidates of every slot from the sweep's normal draws, lane l for
+  // slot l (the R slot's prior depends on d and is formed at its proposal).
+  // The prior changes keep one rounding where the whole expression is one FMA.
+  FDT_DEV void propose(float n) {
+    sxn = sval + n * sprop;
+    sincos_full(sxn, ssn, scn);
+    const bool th = rl >= SL_FIB && (rl - SL_FIB) % 3 == 0;
+    const float lg = lg2(th ? fabsf(ssn) * 0.5f : sxn);
+    const float L = lg * LN2;
+    float p = 0.0f;
+    if (th) p = sxn == 0.0f ? 0.0f : -L;
+    if (MODEL == 3 && rl == SL_D) p = fmaf(sxn, 4000.0f, -(L + L));
+    if (rl == SL_DSTD || (rl == SL_F0 && ardf0)) p = L;
+    sfor<K>([&](auto kc) {
+      if (rl == FK(kc) && can_ard && lam[kc]) p = fudge * L;
+    });
+    sprn = p;
+    sdp = rl == SL_DSTD ? fmaf(lg, LN2, -sprior) : p - sprior;
+    accm = 0;
+  }
+  // end of the sweep: accepted slots take their candidate
+  FDT_DEV void settle() {
+    const bool acc = (accm >> rl) & 1u;
+    scnt += acc ? 1 : rejinc;
+    sval = acc ? sxn : sval;
+    sprior = acc ? sprn : sprior;
+    ssin = acc ? ssn : ssin;
+    scos = acc ? scn : scos;
+  }
+  // lu: log of the uniform draw of the slot.
   // f0 (CUDA/runmcmc_kernels.cu:842-888)
-  FDT_DEV void prop_f0(float n, float lu) {
-    const float f0 = v<SL_F0>();
-    const float f0n = f0 + n * width<SL_F0>();
-    const Fr q = fractions();
-    const float fsn = q.sum - f0 + f0n;
-    if (f0n <= 0.0f || f0n >= 1.0f || fsn > 1.0f) { reject<SL_F0>(); return; }
-    const float prn = ardf0 ? flog(f0n) : 0.0f;
-    const float df = f0n - f0, S0 = v<SL_S0>(), tau = v<SL_TAU>();
-    float a = 0.0f, en[RIC ? VPL : 1];
+  FDT_DEV void prop_f0(float lu) {
+    const float f0n = cand<SL_F0>();
+    const float fsn = fsum - f0 + f0n;
+    if (f0n <= 0.0f || f0n >= 1.0f || fsn > 1.0f) return;
+    const float df = f0n - f0;
+    float a = 0.0f, en[RIC ? VPL : 1], qv[VPL];
     Quad qd;
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
       if (skip(t)) continue;
-      if constexpr (RIC) {
-        en[t] = ell_of(yv(t), S0 * fmaf(df, 1.0f - isov(t), M[t]), tau);
-        a += mask(t, en[t] - ell[t]);
-      } else qd.add(r[t], 1.0f - isov(t));
+      qv[t] = 1.0f - isov(t);
+      if constexpr (!RIC) qd.add(r[t], qv[t]);
     }
+    if constexpr (RIC) ric_terms<false>([&](int t) { return S0 * fmaf(df, qv[t], M[t]); }, tau, en, a);
     a = RIC ? row_sum16(a) : qd.delta(S0 * df);
-    if (dlik(a) + (prn - prior<SL_F0>()) < -lu) {
+    if (dlik(a) + dprior<SL_F0>() < -lu) {
       const float c = S0 * df;
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
         if (skip(t)) continue;
-        const float q = 1.0f - isov(t);
-        M[t] = fmaf(df, q, M[t]);
-        if constexpr (RIC) ell[t] = en[t]; else r[t] = fmaf(-c, q, r[t]);
+        M[t] = fmaf(df, qv[t], M[t]);
+        if constexpr (RIC) ell[t] = en[t]; else r[t] = fmaf(-c, qv[t], r[t]);
       }
       like += (double)a;
-      accept<SL_F0>(f0n, prn);
-    } else reject<SL_F0>();
+      f0 = f0n;
+      fsum = sum_fractions();
+      accept<SL_F0>();
+    }
   }
   // tau (:890-922), Rician only
-  FDT_DEV void prop_tau(float n, float lu) {
+  FDT_DEV void prop_tau(float lu) {
     if constexpr (RIC) {
-      const float tau = v<SL_TAU>();
-      const float tn = tau + n * width<SL_TAU>();
-      if (tn <= 0.0f) { reject<SL_TAU>(); return; }
-      const float S0 = v<SL_S0>();
+      const float tn = cand<SL_TAU>();
+      if (tn <= 0.0f) return;
       float a = 0.0f, yy = 0.0f, en[VPL];
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
-        en[t] = ell_of(yv(t), S0 * M[t], tn);
         const float y = yv(t);
-        a += mask(t, en[t] - ell[t]);
         yy += mask(t, y * y);
       }
+      ric_terms<true>([&](int t) { return S0 * M[t]; }, tn, en, a);
       a = row_sum16(a);  // change of the stored terms (the running sum's)
       // the -tau y^2 / 2 part of the full terms moves with tau too
       float dE = -Nf * (flog(tn) - flog(tau)) - fmaf(-0.5f * (tn - tau), row_sum16(yy), a);
@@ -433,23 +452,23 @@ struct Chain {
 #pragma unroll
         for (int t = 0; t < VPL; ++t) ell[t] = en[t];
         like += (double)a;
-        accept<SL_TAU>(tn, 0.0f);
-      } else reject<SL_TAU>();
+        tau = tn;
+        accept<SL_TAU>();
+      }
     }
   }
   // S0 (:1125-1155)
-  FDT_DEV void prop_S0(float n, float lu) {
-    const float S0 = v<SL_S0>();
-    const float Sn = S0 + n * width<SL_S0>();
-    if (Sn < 0.0f) { reject<SL_S0>(); return; }
-    const float dS = Sn - S0, tau = v<SL_TAU>();
+  FDT_DEV void prop_S0(float lu) {
+    const float Sn = cand<SL_S0>();
+    if (Sn < 0.0f) return;
+    const float dS = Sn - S0;
     float a = 0.0f, en[RIC ? VPL : 1];
     Quad qd;
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
-      if constexpr (RIC) { en[t] = ell_of(yv(t), Sn * M[t], tau); a += mask(t, en[t] - ell[t]); }
-      else qd.add(r[t], mask(t, M[t]));
+      if constexpr (!RIC) qd.add(r[t], mask(t, M[t]));
     }
+    if constexpr (RIC) ric_terms<true>([&](int t) { return Sn * M[t]; }, tau, en, a);
     a = RIC ? row_sum16(a) : qd.delta(dS);
     if (dlik(a) < -lu) {
 #pragma unroll
@@ -457,8 +476,9 @@ struct Chain {
         if constexpr (RIC) ell[t] = en[t]; else r[t] -= dS * mask(t, M[t]);
       }
       like += (double)a;
-      accept<SL_S0>(Sn, 0.0f);
-    } else reject<SL_S0>();
+      S0 = Sn;
+      accept<SL_S0>();
+    }
   }
   // candidate isotropic signal of every shell into the row's table (lane l: shell l)
   template <int SI>
@@ -466,44 +486,6 @@ struct Chain {
     float b = shb[rl];
     isot[rl] = sig<SI>(ci, b, b);
   }
-  // candidate isotropic signal of slot t: from the shell table (SH) or evaluated
-  template <int SI, bool SH>
-  FDT_DEV float iso_new(int t, const SigC& ci, float b) const {
-    if constexpr (SH) return isot[sh[rl + 16 * t]];
-    else return sig<SI>(ci, b, b);
-  }
-  // candidate mixture of slot t when the stick signals (NA) and/or the
-  // isotropic signal (NI) are re-evaluated with coefficients ca / ci
-  // The candidate stick signals are evaluated from b*(g.x_k)^2 and parked in
-  // LDS, so that an accepted move copies them instead of re-evaluating.
-  template <int SA, int SI, bool NA, bool NI, bool SH>
-  FDT_DEV float mix_new(int t, const Fr& q, const SigC& ca, const SigC& ci, const Dirs& D) const {
-    const float4 g = acq[rl + 16 * t];
-    float isn = NI ? iso_new<SI, SH>(t, ci, bv(t, g)) : isov(t);
-    float m = fmaf(1.0f - q.sum, isn, q.f0);
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      float sk = s[k][t];
-      if constexpr (NA) {
-        float dp = fmaf(g.x, D.x[k][0], fmaf(g.y, D.x[k][1], g.z * D.x[k][2]));
-        sk = sig<SA>(ca, g.w * dp * dp, bv(t, g));
-        cnd(k, t) = sk;
-      }
-      m = fmaf(q.fk[k], sk, m);
-    }
-    return m;
-  }
-  template <int SA, int SI, bool NA, bool NI, bool SH>
-  FDT_DEV void store_new(int t, const SigC& ca, const SigC& ci) {
-    float b = bv(t, acq[rl + 16 * t]);
-    if (NI) isov(t) = iso_new<SI, SH>(t, ci, b);
-    if (NA) {
-#pragma unroll
-      for (int k = 0; k < K; ++k) s[k][t] = cnd(k, t);
-    }
-  }
-  // dispatch over the coefficient forms that occur: model 1 (0,0); model 2
-  // (1,1); model 3 sticks 2 with iso 1
   // run f(SH) with SH = true when the isotropic signal changes and the
   // acquisition has a shell table (the loop over slots is then the table
   // variant only; no per-slot branch)
@@ -514,184 +496,235 @@ struct Chain {
       else f(std::false_type{});
     } else f(std::false_type{});
   }
-  template <class F>
-  FDT_DEV void by_forms(const SigC& ca, const SigC& ci, bool na, bool ni, F&& f) const {
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    using T_ = std::true_type;
-    using F_ = std::false_type;
-    // the isotropic form is kind 0 for model 1 and kind 1 otherwise
-    if (na && ni) {
-      if (ca.kind == 0) f(I0{}, I0{}, T_{}, T_{});
-      else if (ca.kind == 1) f(I1{}, I1{}, T_{}, T_{});
-      else f(I2{}, I1{}, T_{}, T_{});
-    } else if (ni) {
-      f(I0{}, I1{}, F_{}, T_{});
-    } else {
-      f(I2{}, I0{}, T_{}, F_{});
+  // the Rician terms of every slot at the signals p(t) and precision tv into
+  // en[], and their change into a.  Both series of log I0 cost 26 operations,
+  // the one above 3.75 alone 14; x = tau p y is ~SNR^2, so most slots of most
+  // waves need only that one: a vote over each group of slots takes it where
+  // no volume of the wave is below 3.75 (the results are the same).
+  static constexpr int RG = 3;
+  // ALL: also slot 0 of b = 0 volumes (the S0 and tau moves).
+  template <bool ALL, class P>
+  FDT_DEV void ric_terms(P&& p, float tv, float (&en)[RIC ? VPL : 1], float& a) const {
+#pragma unroll
+    for (int t0 = 0; t0 < VPL; t0 += RG) {
+      float q[RG], x[RG];
+      bool sm = false;
+      auto out = [&](int t) { return t >= VPL || (!ALL && skip(t)); };
+#pragma unroll
+      for (int i = 0; i < RG; ++i) {
+        const int t = t0 + i;
+        q[i] = x[i] = 0.0f;
+        if (out(t)) continue;
+        q[i] = p(t);
+        x[i] = tv * q[i] * yv(t);
+        sm = sm || (t < nv && fabsf(x[i]) < 3.75f);
+      }
+      if (__builtin_amdgcn_ballot_w64(sm)) {
+#pragma unroll
+        for (int i = 0; i < RG; ++i)
+          if (t0 + i < VPL) x[i] = logI0f(x[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < RG; ++i)
+          if (t0 + i < VPL) x[i] = logI0_large(x[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < RG; ++i) {
+        const int t = t0 + i;
+        if (out(t)) continue;
+        en[t] = fmaf(-0.5f * (tv * q[i]), q[i], x[i]);
+        a += mask(t, en[t] - ell[t]);
+      }
     }
   }
   // all stick signals and/or iso change: d (:924-985), d_std (:987-1051), R
-  // (:1053-1122).  The row sum of the likelihood change is accumulated on the
-  // fly; the candidate stick signals go to the wave's LDS block (mix_new) and
-  // an accepted move copies them back (store_new), re-evaluating only the
-  // isotropic signal, so the live registers stay the chain state.
+  // (:1053-1122).  NA: the stick signals change, NI: the isotropic signal.
   template <int SL>
-  FDT_DEV void prop_global(float n, float lu) {
-    const float d = v<SL_D>(), dstd = v<SL_DSTD>(), Rr = v<SL_R>();
-    float dn = d, dsn = dstd, Rn = Rr, prn = 0.0f, xn;
-    bool new_aniso = true, new_iso = true;
+  FDT_DEV void prop_global(float lu) {
+    constexpr bool NA = !(SL == SL_DSTD && MODEL == 3), NI = SL != SL_R;
+    constexpr int SA = STICK_KIND<MODEL>, SI = ISO_KIND<MODEL>;
+    float dn = d, dsn = dstd, Rn = Rr;
     if constexpr (SL == SL_D) {
-      dn = xn = d + n * width<SL>();
-      if (dn < 0.0f || dn > UPPERDIFF_F) { reject<SL>(); return; }
-      prn = model == 3 ? (1.0f - 3.0f) * flog(dn) + 4000.0f * dn : 0.0f;
+      dn = cand<SL>();
+      if (dn < 0.0f || dn > UPPERDIFF_F) return;
     } else if constexpr (SL == SL_DSTD) {
-      dsn = xn = dstd + n * width<SL>();
-      float up = model == 3 ? 0.004f : 0.01f;
-      if (dsn <= 0.0f || dsn > up) { reject<SL>(); return; }
-      prn = flog(dsn);
-      new_aniso = (model == 2);
+      dsn = cand<SL>();
+      if (dsn <= 0.0f || dsn > (MODEL == 3 ? 0.004f : 0.01f)) return;
     } else {
-      Rn = xn = Rr + n * width<SL>();
-      if (!r_prior(Rn, d, prn)) { reject<SL>(); return; }
-      new_iso = false;
+      Rn = cand<SL>();
+      float prn = 0.0f;
+      if (!r_prior(Rn, d, prn)) return;
+      if (rl == SL_R) { sprn = prn; sdp = prn - sprior; }
     }
-    const SigC ca = aniso_coef(model, dn, dsn, Rn), ci = iso_coef(model, dn, dsn);
-    const Fr q = fractions();
-    const Dirs D = new_aniso ? dirs() : Dirs{};
-    const float S0 = v<SL_S0>(), tau = v<SL_TAU>();
+    const SigC cn = aniso_coef<MODEL>(dn, dsn, Rn), ci = iso_coef<MODEL>(dn, dsn);
     reload_acq();
-    float a = 0.0f;
+    constexpr bool KEEP_M = U_LDS || RIC;
+    float a = 0.0f, mn[KEEP_M ? VPL : 1], en[RIC ? VPL : 1], sn[U_LDS ? K : 1][VPL];
+    Dirs D;
+    if constexpr (NA && !U_LDS) D = dirs();
     Quad qd;
-    by_forms(ca, ci, new_aniso, new_iso, [&](auto SA, auto SI, auto NA, auto NI) {
-      by_shells<decltype(NI)::value>([&](auto SH) {
-        if constexpr (decltype(SH)::value) fill_iso<decltype(SI)::value>(ci);
+    by_shells<NI>([&](auto SHc) {
+      constexpr bool SH = decltype(SHc)::value;
+      if constexpr (SH) fill_iso<SI>(ci);
+      // slot t's reads are issued one slot ahead (the shell index two), so
+      // that they return while the slot before it computes
+      float u[NA && U_LDS ? K : 1][VPL], iso[VPL], b[VPL];
+      float4 g[NA && !U_LDS ? VPL : 1];
+      int si[SH ? VPL : 1];
+      auto index = [&](int t) {
+        if constexpr (SH) { if (t < VPL) si[t] = sh[rl + 16 * t]; }
+      };
+      auto fetch = [&](int t) {
+        if (t >= VPL) return;
+        if constexpr (NA && U_LDS) {
+#pragma unroll
+          for (int k = 0; k < K; ++k) u[k][t] = ldsk(k, t);
+        }
+        if constexpr (NA && !U_LDS) g[t] = acq[rl + 16 * t];
+        if constexpr ((NA && SA == 2) || (NI && !SH)) b[t] = bv(t, acq[rl + 16 * t]);
+        if constexpr (SH) iso[t] = isot[si[t]];
+        else if constexpr (!NI) iso[t] = isov(t);
+      };
+      index(0);
+      index(1);
+      fetch(0);
+#pragma unroll
+      for (int t = 0; t < VPL; ++t) {
+        index(t + 2);
+        fetch(t + 1);
+        if (skip(t)) continue;
+        if constexpr (NI && !SH) iso[t] = sig<SI>(ci, b[t], b[t]);
+        float m = fmaf(1.0f - fsum, iso[t], f0);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          float sk_ = s[k][t];
+          if constexpr (NA && U_LDS) sk_ = sn[k][t] = sig<SA>(cn, u[k][t], b[t]);
+          if constexpr (NA && !U_LDS) {
+            const float dp = fmaf(g[t].x, D.x[k][0], fmaf(g[t].y, D.x[k][1], g[t].z * D.x[k][2]));
+            ldsk(k, t) = sk_ = sig<SA>(cn, g[t].w * dp * dp, b[t]);
+          }
+          m = fmaf(fk[k], sk_, m);
+        }
+        if constexpr (KEEP_M) mn[t] = m;
+        if constexpr (!RIC) qd.add(r[t], mask(t, m - M[t]));
+        // the gamma form has several temporaries per volume and signal: keep
+        // the scheduler from overlapping many volumes of it (register spills)
+        if constexpr ((NA && SA == 1) || (NI && SI == 1)) reload_acq();
+      }
+    });
+    if constexpr (RIC) ric_terms<false>([&](int t) { return S0 * mn[t]; }, tau, en, a);
+    a = RIC ? row_sum16(a) : qd.delta(S0);
+    if (dlik(a) + dprior<SL>() < -lu) {
+      reload_acq();
+      by_shells<NI>([&](auto SHc) {
 #pragma unroll
         for (int t = 0; t < VPL; ++t) {
           if (skip(t)) continue;
-          float mn = mix_new<decltype(SA)::value, decltype(SI)::value, decltype(NA)::value, decltype(NI)::value,
-                             decltype(SH)::value>(t, q, ca, ci, D);
-          if constexpr (RIC) a += mask(t, ell_of(yv(t), S0 * mn, tau) - ell[t]);
-          else qd.add(r[t], mask(t, mn - M[t]));
-          // the gamma form has several temporaries per volume and signal: keep
-          // the scheduler from overlapping many volumes of it (register spills)
-          if constexpr (decltype(SA)::value == 1 || decltype(SI)::value == 1) reload_acq();
+          if constexpr (NI) {
+            if constexpr (decltype(SHc)::value) isov(t) = isot[sh[rl + 16 * t]];
+            else {
+              const float b = bv(t, acq[rl + 16 * t]);
+              isov(t) = sig<SI>(ci, b, b);
+            }
+          }
+          if constexpr (NA) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) s[k][t] = U_LDS ? sn[U_LDS ? k : 0][t] : ldsk(k, t);
+          }
         }
       });
-    });
-    a = RIC ? row_sum16(a) : qd.delta(S0);
-    if (dlik(a) + (prn - prior<SL>()) < -lu) {
-      // store the new signals, then form the mixture from them with the
-      // same expression as the candidate (bit-identical to it)
-      reload_acq();
-      by_forms(ca, ci, new_aniso, new_iso, [&](auto SA, auto SI, auto NA, auto NI) {
-        by_shells<decltype(NI)::value>([&](auto SH) {
-#pragma unroll
-          for (int t = 0; t < VPL; ++t) {
-            if (skip(t)) continue;
-            store_new<decltype(SA)::value, decltype(SI)::value, decltype(NA)::value, decltype(NI)::value,
-                      decltype(SH)::value>(t, ca, ci);
-            float mn = mix(t, q);
-            if constexpr (RIC) ell[t] = ell_of(yv(t), S0 * mn, tau); else r[t] -= S0 * mask(t, mn - M[t]);
-            M[t] = mn;
-          }
-        });
-      });
-      like += (double)a;
-      accept<SL>(xn, prn);
-      set_aniso_cache(ca);
-    } else reject<SL>();
-  }
-  // theta_k / phi_k (:1157-1265); the theta prior lives in the theta slot
-  template <int k, bool IS_TH>
-  FDT_DEV void prop_angle(float n, float lu) {
-    constexpr int SL = IS_TH ? TH(k) : PH(k);
-    constexpr int SO = IS_TH ? PH(k) : TH(k);  // the other angle's slot: its sin/cos are cached there
-    const float xn = v<SL>() + n * width<SL>();
-    float sn_, cn_;
-    sincos_full(xn, sn_, cn_);
-    const float so = row_bcast<SO>(ssin), co = row_bcast<SO>(scos);
-    float prn = 0.0f, prold = 0.0f;
-    if constexpr (IS_TH) { prn = theta_prior(xn, sn_); prold = prior<SL>(); }
-    const float st = IS_TH ? sn_ : so, ct = IS_TH ? cn_ : co;
-    const float sp = IS_TH ? so : sn_, cp = IS_TH ? co : cn_;
-    float x0 = st * cp, x1 = st * sp, x2 = ct;
-    xform(x0, x1, x2);
-    const SigC ca = aniso_cached();
-    const float fk = v<FK(k)>(), S0 = v<SL_S0>(), tau = v<SL_TAU>();
-    reload_acq();
-    float sn[VPL], en[RIC ? VPL : 1];
-    float a = 0.0f;
-    by_kind(ca.kind, [&](auto SK) {
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
         if (skip(t)) continue;
-        float4 g = acq[rl + 16 * t];
-        float dp = fmaf(g.x, x0, fmaf(g.y, x1, g.z * x2));
-        sn[t] = sig<decltype(SK)::value>(ca, g.w * dp * dp, bv(t, g));
+        const float m = KEEP_M ? mn[KEEP_M ? t : 0] : mix(t);  // mix(t) repeats the candidate's expression
+        if constexpr (RIC) ell[t] = en[t]; else r[t] -= S0 * mask(t, m - M[t]);
+        M[t] = m;
       }
-    });
+      like += (double)a;
+      if constexpr (SL == SL_D) d = dn;
+      else if constexpr (SL == SL_DSTD) dstd = dsn;
+      else Rr = Rn;
+      ca = cn;
+      accept<SL>();
+    }
+  }
+  // theta_k / phi_k (:1157-1265); st..cp: sin and cos of fibre k's current
+  // angles, updated with an accepted move
+  template <int k, bool IS_TH>
+  FDT_DEV void prop_angle(float lu, float& st, float& ct, float& sp, float& cp) {
+    constexpr int SL = IS_TH ? TH(k) : PH(k);
+    const float sa = row_bcast<SL>(ssn), cs = row_bcast<SL>(scn);
+    const float st_ = IS_TH ? sa : st, ct_ = IS_TH ? cs : ct;
+    const float sp_ = IS_TH ? sp : sa, cp_ = IS_TH ? cp : cs;
+    float x0 = st_ * cp_, x1 = st_ * sp_, x2 = ct_;
+    xform(x0, x1, x2);
+    reload_acq();
+    float sn[VPL], un[U_LDS ? VPL : 1], qv[VPL], en[RIC ? VPL : 1];
+    float a = 0.0f;
+#pragma unroll
+    for (int t = 0; t < VPL; ++t) {
+      if (skip(t)) continue;
+      float4 g = acq[rl + 16 * t];
+      float dp = fmaf(g.x, x0, fmaf(g.y, x1, g.z * x2));
+      const float u = g.w * dp * dp;
+      if constexpr (U_LDS) un[t] = u;
+      sn[t] = sig<STICK_KIND<MODEL>>(ca, u, bv(t, g));
+    }
     Quad qd;
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
       if (skip(t)) continue;
-      if constexpr (RIC) {
-        en[t] = ell_of(yv(t), S0 * fmaf(fk, sn[t] - s[k][t], M[t]), tau);
-        a += mask(t, en[t] - ell[t]);
-      } else qd.add(r[t], sn[t] - s[k][t]);
+      qv[t] = sn[t] - s[k][t];
+      if constexpr (!RIC) qd.add(r[t], qv[t]);
     }
-    a = RIC ? row_sum16(a) : qd.delta(S0 * fk);
-    if (dlik(a) + (prn - prold) < -lu) {
-      reload_acq();
-      const float c = S0 * fk;
+    if constexpr (RIC) ric_terms<false>([&](int t) { return S0 * fmaf(fk[k], qv[t], M[t]); }, tau, en, a);
+    a = RIC ? row_sum16(a) : qd.delta(S0 * fk[k]);
+    if (dlik(a) + (IS_TH ? dprior<SL>() : 0.0f) < -lu) {
+      const float c = S0 * fk[k];
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
         if (skip(t)) continue;
-        const float q = sn[t] - s[k][t];
-        M[t] = fmaf(fk, q, M[t]);
-        if constexpr (RIC) ell[t] = en[t]; else r[t] = fmaf(-c, q, r[t]);
+        M[t] = fmaf(fk[k], qv[t], M[t]);
+        if constexpr (RIC) ell[t] = en[t]; else r[t] = fmaf(-c, qv[t], r[t]);
         s[k][t] = sn[t];
+        if constexpr (U_LDS) ldsk(k, t) = un[t];
       }
       like += (double)a;
-      if (rl == SL) { ssin = sn_; scos = cn_; }
-      if constexpr (IS_TH) accept<SL>(xn, prn);
-      else if (rl == SL) { sval = xn; scnt += 1; }
-    } else reject<SL>();
+      if constexpr (IS_TH) { st = sa; ct = cs; } else { sp = sa; cp = cs; }
+      accept<SL>();
+    }
   }
   // f_k (:1267-1322)
   template <int k>
-  FDT_DEV void prop_f(float n, float lu) {
+  FDT_DEV void prop_f(float lu) {
     constexpr int SL = FK(k);
-    const Fr q = fractions();
-    const float fn = q.fk[k] + n * width<SL>();
-    const float fsn = q.sum - q.fk[k] + fn;
-    if (fn <= 0.0f || fn >= 1.0f || fsn > 1.0f) { reject<SL>(); return; }
-    const float prn = (can_ard && lam[k]) ? fudge * flog(fn) : 0.0f;
-    const float df = fn - q.fk[k], S0 = v<SL_S0>(), tau = v<SL_TAU>();
-    float a = 0.0f, en[RIC ? VPL : 1];
+    const float fn = cand<SL>();
+    const float fsn = fsum - fk[k] + fn;
+    if (fn <= 0.0f || fn >= 1.0f || fsn > 1.0f) return;
+    const float df = fn - fk[k];
+    float a = 0.0f, en[RIC ? VPL : 1], qv[VPL];
     Quad qd;
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
       if (skip(t)) continue;
-      if constexpr (RIC) {
-        en[t] = ell_of(yv(t), S0 * fmaf(df, s[k][t] - isov(t), M[t]), tau);
-        a += mask(t, en[t] - ell[t]);
-      } else qd.add(r[t], s[k][t] - isov(t));
+      qv[t] = s[k][t] - isov(t);
+      if constexpr (!RIC) qd.add(r[t], qv[t]);
     }
+    if constexpr (RIC) ric_terms<false>([&](int t) { return S0 * fmaf(df, qv[t], M[t]); }, tau, en, a);
     a = RIC ? row_sum16(a) : qd.delta(S0 * df);
-    if (dlik(a) + (prn - prior<SL>()) < -lu) {
+    if (dlik(a) + dprior<SL>() < -lu) {
       const float c = S0 * df;
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
         if (skip(t)) continue;
-        const float q = s[k][t] - isov(t);
-        M[t] = fmaf(df, q, M[t]);
-        if constexpr (RIC) ell[t] = en[t]; else r[t] = fmaf(-c, q, r[t]);
+        M[t] = fmaf(df, qv[t], M[t]);
+        if constexpr (RIC) ell[t] = en[t]; else r[t] = fmaf(-c, qv[t], r[t]);
       }
       like += (double)a;
-      accept<SL>(fn, prn);
-    } else reject<SL>();
+      fk[k] = fn;
+      fsum = sum_fractions();
+      accept<SL>();
+    }
   }
 
   // proposal-width adaptation every upe jumps (:1341-1395), all slots of the
@@ -705,12 +738,12 @@ struct Chain {
   }
 };
 
-// LDS of a chain workgroup: the acquisition table, candidate stick signals per wave, the
+// LDS of a chain workgroup: the acquisition table, the stick-signal arguments per wave, the
 // b-shell index of each volume and the shells' b values, the rows' isotropic
 // shell tables
 struct ChainLds {
   float4* acq;
-  float* cand;
+  float* sk;
   int* sh;     // null without a shell table (--gradnonlin)
   float* shb;
   float* iso;
@@ -798,16 +831,16 @@ FDT_DEV bool zero_slot0(const ChainLds& L) {
 // :507-1474, run twice by CUDA/runmcmc.cu:108-316).  GN (--gradnonlin): the
 // chain reads its voxel's own corrected acquisition from a.acqv (the reference
 // indexes per-voxel bvals/alpha/beta with posBV, :266, :711).
-template <int K, int VPL, bool RIC, bool GN = false>
+template <int K, int VPL, int MODEL, bool RIC, bool GN = false>
 FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
-  using C = Chain<K, VPL, RIC, GN>;
+  using C = Chain<K, VPL, MODEL, RIC, GN>;
   const int lane = __lane_id();
   const int rl = lane & 15;
   const float4* sacq = L.acq;
   C c;
   c.rl = rl;
   c.acq = sacq;
-  c.cand = L.cand + (threadIdx.x >> 6) * (K * VPL * 64) + lane;
+  c.sk = L.sk + (threadIdx.x >> 6) * (K * VPL * 64) + lane;
   c.vol = L.vol ? L.vol + (threadIdx.x >> 6) * (VPL * 64) + lane : nullptr;
   c.sh = L.sh;
   c.shb = L.shb;
@@ -828,7 +861,6 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
     c.bp = bp;
     c.gd = gd;
   }
-  c.model = a.model;
   c.incf0 = a.f0 != 0;
   c.ardf0 = a.ardf0 != 0;
   c.can_ard = a.no_ard == 0;
@@ -867,15 +899,15 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
   // ---- chain initialisation (init_Fibres_Multifibres_kernel, :265-504):
   // every lane loads the parameter of its slot and evaluates its prior
   const float* P = a.params + (size_t)vox * a.np;
-  const int add = a.model >= 2 ? 1 : 0;
+  const int add = MODEL >= 2 ? 1 : 0;
   float d = P[1];
   if (d < 0.0f || d > UPPERDIFF_F) d = 2e-3f;
   float dstd = 0.0f, Rr = 0.0f;
-  if (a.model >= 2) {
+  if (MODEL >= 2) {
     dstd = P[2];
-    float up = a.model == 3 ? 0.004f : 0.01f;
+    float up = MODEL == 3 ? 0.004f : 0.01f;
     if (dstd < 0.0f || dstd > up) dstd = d / 10.0f;
-    if (a.model == 3) Rr = a.Rmean;
+    if (MODEL == 3) Rr = a.Rmean;
   }
   float val = 0.0f, pr = 0.0f, wd = 0.2f;  // f0 and the fibre slots start at width 0.2 (:497-503)
   float vs = 0.0f, vc = 1.0f;              // sin / cos of an angle slot's value
@@ -887,17 +919,17 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
     wd = val / 2.0f;
   } else if (rl == SL_D) {
     val = d;
-    if (a.model == 3) pr = (1.0f - 3.0f) * flog(d) + 4000.0f * d;
+    if (MODEL == 3) pr = (1.0f - 3.0f) * flog(d) + 4000.0f * d;
     wd = d / 10.0f;
   } else if (rl == SL_DSTD) {
     val = dstd;
-    float up = a.model == 3 ? 0.004f : 0.01f;
-    if (a.model >= 2 && dstd > 0.0f && dstd <= up) pr = flog(dstd);
+    float up = MODEL == 3 ? 0.004f : 0.01f;
+    if (MODEL >= 2 && dstd > 0.0f && dstd <= up) pr = flog(dstd);
     wd = dstd / 10.0f;
   } else if (rl == SL_R) {
     val = Rr;
     float q;
-    if (a.model == 3 && c.r_prior(Rr, d, q)) pr = q;
+    if (MODEL == 3 && c.r_prior(Rr, d, q)) pr = q;
     wd = Rr / 10.0f;
   } else if (rl == SL_S0) {
     val = P[0];
@@ -922,25 +954,33 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
   c.ssin = vs;
   c.scos = vc;
   c.scnt = 0;
+  c.rejinc = 0;
+  if (rl == SL_D || rl == SL_S0 || (rl >= SL_FIB && rl < SL_FIB + 3 * K) || (rl == SL_F0 && c.incf0) ||
+      (rl == SL_TAU && RIC) || (rl == SL_DSTD && MODEL >= 2) || (rl == SL_R && MODEL == 3))
+    c.rejinc = 1 << 16;
+  c.S0 = row_bcast<SL_S0>(val);
+  c.tau = row_bcast<SL_TAU>(val);
+  c.d = d; c.dstd = dstd; c.Rr = Rr;
+  c.f0 = row_bcast<SL_F0>(val);
+  sfor<K>([&](auto kc) { c.fk[kc] = row_bcast<C::FK(kc)>(val); });
+  c.fsum = c.sum_fractions();
   {
-    SigC ca = aniso_coef(a.model, d, dstd, Rr), ci = iso_coef(a.model, d, dstd);
-    c.set_aniso_cache(ca);
+    c.ca = aniso_coef<MODEL>(d, dstd, Rr);
+    const SigC ci = iso_coef<MODEL>(d, dstd);
     const typename C::Dirs D = c.dirs();
-    by_kind(ca.kind, [&](auto SK) {
 #pragma unroll
-      for (int t = 0; t < VPL; ++t) {
-        float4 g = sacq[rl + 16 * t];
+    for (int t = 0; t < VPL; ++t) {
+      float4 g = sacq[rl + 16 * t];
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-          float dp = fmaf(g.x, D.x[k][0], fmaf(g.y, D.x[k][1], g.z * D.x[k][2]));
-          c.s[k][t] = sig<decltype(SK)::value>(ca, g.w * dp * dp, c.bv(t, g));
-        }
+      for (int k = 0; k < K; ++k) {
+        float dp = fmaf(g.x, D.x[k][0], fmaf(g.y, D.x[k][1], g.z * D.x[k][2]));
+        const float u = g.w * dp * dp;
+        if constexpr (C::U_LDS) c.ldsk(k, t) = u;
+        c.s[k][t] = sig<STICK_KIND<MODEL>>(c.ca, u, c.bv(t, g));
       }
-    });
-    by_kind(ci.kind, [&](auto SK) {
+    }
 #pragma unroll
-      for (int t = 0; t < VPL; ++t) { float b = c.bv(t, sacq[rl + 16 * t]); c.isov(t) = sig<decltype(SK)::value>(ci, b, b); }
-    });
+    for (int t = 0; t < VPL; ++t) { float b = c.bv(t, sacq[rl + 16 * t]); c.isov(t) = sig<ISO_KIND<MODEL>>(ci, b, b); }
   }
   if constexpr (RIC) {
 #pragma unroll
@@ -972,20 +1012,24 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
   for (int j = 0; j < total; ++j) {
     float nl, lul;
     draw(a.seed, gvox, (uint32_t)j, (uint32_t)rl, nl, lul);
-    if (c.incf0) c.prop_f0(row_bcast<SL_F0>(nl), row_bcast<SL_F0>(lul));
-    if (RIC) c.prop_tau(row_bcast<SL_TAU>(nl), row_bcast<SL_TAU>(lul));
-    c.template prop_global<SL_D>(row_bcast<SL_D>(nl), row_bcast<SL_D>(lul));
-    if (a.model >= 2) {
-      c.template prop_global<SL_DSTD>(row_bcast<SL_DSTD>(nl), row_bcast<SL_DSTD>(lul));
-      if (a.model == 3) c.template prop_global<SL_R>(row_bcast<SL_R>(nl), row_bcast<SL_R>(lul));
+    c.propose(nl);
+    if (c.incf0) c.prop_f0(row_bcast<SL_F0>(lul));
+    if (RIC) c.prop_tau(row_bcast<SL_TAU>(lul));
+    c.template prop_global<SL_D>(row_bcast<SL_D>(lul));
+    if (MODEL >= 2) {
+      c.template prop_global<SL_DSTD>(row_bcast<SL_DSTD>(lul));
+      if (MODEL == 3) c.template prop_global<SL_R>(row_bcast<SL_R>(lul));
     }
-    c.prop_S0(row_bcast<SL_S0>(nl), row_bcast<SL_S0>(lul));
+    c.prop_S0(row_bcast<SL_S0>(lul));
     sfor<K>([&](auto kc) {
       constexpr int k = kc;
-      c.template prop_angle<k, true>(row_bcast<C::TH(k)>(nl), row_bcast<C::TH(k)>(lul));
-      c.template prop_angle<k, false>(row_bcast<C::PH(k)>(nl), row_bcast<C::PH(k)>(lul));
-      c.template prop_f<k>(row_bcast<C::FK(k)>(nl), row_bcast<C::FK(k)>(lul));
+      float st = row_bcast<C::TH(k)>(c.ssin), ct = row_bcast<C::TH(k)>(c.scos);
+      float sp = row_bcast<C::PH(k)>(c.ssin), cp = row_bcast<C::PH(k)>(c.scos);
+      c.template prop_angle<k, true>(row_bcast<C::TH(k)>(lul), st, ct, sp, cp);
+      c.template prop_angle<k, false>(row_bcast<C::PH(k)>(lul), st, ct, sp, cp);
+      c.template prop_f<k>(row_bcast<C::FK(k)>(lul));
     });
+    c.settle();
 
     // record: the lane of each sampled slot writes its value
     if (j >= a.nburn) {
@@ -1015,7 +1059,7 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
     }
   }
   if (a.energy) {
-    const float tau = c.template v<SL_TAU>();
+    const float tau = c.tau;
     double e = c.like;
     if constexpr (RIC) {
       double sl = 0.0, sy = 0.0;  // the model-independent part of the Rician terms
@@ -1032,7 +1076,7 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
   if (a.ssr) {  // sum of squares of the final state's residuals (the Rician chain keeps the data in r)
     double ss;
     if constexpr (RIC) {
-      const float S0 = c.template v<SL_S0>();
+      const float S0 = c.S0;
       float acc = 0.0f;
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {

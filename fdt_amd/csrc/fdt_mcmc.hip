@@ -15,7 +15,7 @@ __device__ inline int xcd_tile(int b, int nb) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + l;
 }
 
-template <int K, int VPL, bool RIC, bool GN>
+template <int K, int VPL, int MODEL, bool RIC, bool GN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VPL <= 18 ? 2 : 1, 2))) void mcmc_kernel(McmcArgs a) {
   __shared__ float4 sacq[16 * VPL];
   __shared__ float sba[4 * K * VPL * 64];
@@ -33,15 +33,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VPL <= 18 ?
   stage_acq<VPL>(a, L);
   __syncthreads();
   const int i = xcd_tile(blockIdx.x, gridDim.x) * 16 + (threadIdx.x >> 4);
-  if (i < a.nvox) run_chain<K, VPL, RIC, GN>(a, a.list ? a.list[i] : i, L);
+  if (i < a.nvox) run_chain<K, VPL, MODEL, RIC, GN>(a, a.list ? a.list[i] : i, L);
 }
 
 }  // namespace fdt
 
 // Two translation units per VPL value (-DFDT_VPL=...): -DFDT_MCMC_RIC=0 holds
 // the Gaussian kernels and the launcher, -DFDT_MCMC_RIC=1 the Rician ones
-// (built in parallel; each can take its own compiler options).  K = 1..3, with the shared
-// acquisition or per-voxel ones (--gradnonlin, a->acqv set; its stride must
+// (built in parallel; each can take its own compiler options).  K = 1..3 and
+// models 1..3 (a kernel each: one that held all models at once took 128 KB of code at K = 3 and 98 scalar
+// registers more than there are), with the shared acquisition or per-voxel ones (--gradnonlin, a->acqv set; its stride must
 // cover 16 * VPL volumes).
 #ifndef FDT_VPL
 #define FDT_VPL 18
@@ -51,28 +52,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VPL <= 18 ?
 #endif
 #define FDT_CAT2_(a, b) a##b
 #define FDT_CAT2(a, b) FDT_CAT2_(a, b)
-#define FDT_MC_CASE(KK, RR, GG) \
-  if (K == KK && gn == GG) { hipLaunchKernelGGL((fdt::mcmc_kernel<KK, FDT_VPL, RR, GG>), grid, block, 0, s, *a); return hipGetLastError(); }
+
+namespace {
+template <int K, int MODEL, bool RIC>
+hipError_t launch_model(const fdt::McmcArgs* a, hipStream_t s) {
+  dim3 grid((a->nvox + 15) / 16), block(256);
+  if (a->acqv) hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, true>), grid, block, 0, s, *a);
+  else hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false>), grid, block, 0, s, *a);
+  return hipGetLastError();
+}
+template <int K, bool RIC>
+hipError_t launch_k(const fdt::McmcArgs* a, hipStream_t s) {
+  if (a->model == 1) return launch_model<K, 1, RIC>(a, s);
+  if (a->model == 2) return launch_model<K, 2, RIC>(a, s);
+  if (a->model == 3) return launch_model<K, 3, RIC>(a, s);
+  return hipErrorInvalidValue;
+}
+template <bool RIC>
+hipError_t launch(const fdt::McmcArgs* a, int K, hipStream_t s) {
+  if (K == 1) return launch_k<1, RIC>(a, s);
+  if (K == 2) return launch_k<2, RIC>(a, s);
+  if (K == 3) return launch_k<3, RIC>(a, s);
+  return hipErrorInvalidValue;
+}
+}  // namespace
 
 #if FDT_MCMC_RIC
 extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, hipStream_t s) {
-  dim3 grid((a->nvox + 15) / 16), block(256);
-  const bool gn = a->acqv != nullptr;
-  FDT_MC_CASE(1, true, false) FDT_MC_CASE(2, true, false) FDT_MC_CASE(3, true, false)
-  FDT_MC_CASE(1, true, true) FDT_MC_CASE(2, true, true) FDT_MC_CASE(3, true, true)
-  return hipErrorInvalidValue;
+  return launch<true>(a, K, s);
 }
 #else
 extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, hipStream_t s);
 extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, int rician, hipStream_t s) {
   if (a->nvox <= 0) return hipSuccess;
   if (a->acqv && a->acqv_stride < 16 * FDT_VPL) return hipErrorInvalidValue;
-  if (rician) return FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(a, K, s);
-  dim3 grid((a->nvox + 15) / 16), block(256);
-  const bool gn = a->acqv != nullptr;
-  FDT_MC_CASE(1, false, false) FDT_MC_CASE(2, false, false) FDT_MC_CASE(3, false, false)
-  FDT_MC_CASE(1, false, true) FDT_MC_CASE(2, false, true) FDT_MC_CASE(3, false, true)
-  return hipErrorInvalidValue;
+  return rician ? FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(a, K, s) : launch<false>(a, K, s);
 }
 #endif
-#undef FDT_MC_CASE

@@ -17,7 +17,10 @@ template <int K, int VPL>
 FDT_DEV void queue_item(const McmcArgs& a, int vox, bool active, const ChainLds& L) {
   stage_acq<VPL>(a, L);
   __syncthreads();
-  if (active) run_chain<K, VPL, false>(a, vox, L);
+  if (!active) return;
+  if (a.model == 1) run_chain<K, VPL, 1, false>(a, vox, L);
+  else if (a.model == 2) run_chain<K, VPL, 2, false>(a, vox, L);
+  else run_chain<K, VPL, 3, false>(a, vox, L);
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void mcmc_queue_kernel(QueueArgs q) {
