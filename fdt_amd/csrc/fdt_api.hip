@@ -39,11 +39,11 @@ hipError_t fdt_launch_f0_flag(const F0FlagArgs*, hipStream_t);
 hipError_t fdt_launch_zero_ints(int*, int, hipStream_t);
 hipError_t fdt_launch_mcmc_queue(const QueueArgs*, int rows_per_wg, int max_items, hipStream_t);
 hipError_t fdt_launch_gemm_bf16(const GemmArgs*, hipStream_t);
-hipError_t fdt_launch_mlp_ew(int op, const void* a, const void* b, void* c, size_t n, int M, int N, hipStream_t);
+hipError_t fdt_launch_to_bf16(const float* x, uint16_t* y, size_t n, hipStream_t);
 hipError_t fdt_launch_adam(float* w, float* m, float* v, const float* g, uint16_t* wb, size_t n, float lr, float b1,
                            float b2, float eps, int step, hipStream_t);
 hipError_t fdt_launch_normalize(const float* data, int N, int nvox, const float* bvals, float b0_max, uint16_t* X,
-                                float* S0, hipStream_t);
+                                int ldx, float* S0, hipStream_t);
 hipError_t fdt_launch_sg_loss(const float* O, const float* T, int M, uint16_t* dO, float* loss_part, float w_lw,
                               hipStream_t);
 hipError_t fdt_launch_sg_decode(const SgDecodeArgs*, hipStream_t);
@@ -1483,21 +1483,20 @@ int fdt_queue_autotune(fdt_queue* q, int jumps, int sample_vox, float* ms_best) 
 struct fdt_surrogate {
   int device = 0;
   hipStream_t stream = nullptr;
-  int n_in = 0;
+  int n_in = 0, ldx = 0;  // ldx: row length of the normalised signals (whole 16-byte units)
   int dims[SG_LAYERS + 1] = {};
   size_t woff[SG_LAYERS] = {}, boff[SG_LAYERS] = {}, nw = 0;
   DevBuf<float> w, m, v, g;
   DevBuf<uint16_t> wb;
   int step = 0;
-  DevBuf<uint16_t> X;  // normalised training signals [n][n_in]
+  DevBuf<uint16_t> X;  // normalised training signals [n][ldx]
   DevBuf<float> T;     // targets [n][SG_OUT]
   DevBuf<float> bvals;
   int ntrain = 0;
   int cap = 0;  // batch capacity of the activation buffers
   DevBuf<float> Z[SG_LAYERS];
   DevBuf<uint16_t> A[SG_LAYERS];
-  DevBuf<float> dA;
-  DevBuf<uint16_t> dZ, Xb;
+  DevBuf<uint16_t> dZ[2], Xb;
   DevBuf<float> loss_part, S0;
   std::string err;
 };
@@ -1523,36 +1522,40 @@ static int sg_reserve(fdt_surrogate* s, int b) {
     SHIP(s, s->Z[l].ensure((size_t)b * s->dims[l + 1]));
     SHIP(s, s->A[l].ensure((size_t)b * s->dims[l + 1]));
   }
-  SHIP(s, s->dA.ensure((size_t)b * 512));
-  SHIP(s, s->dZ.ensure((size_t)b * 512));
-  SHIP(s, s->Xb.ensure((size_t)b * s->n_in));
+  for (auto& d : s->dZ) SHIP(s, d.ensure((size_t)b * 512));
+  SHIP(s, s->Xb.ensure((size_t)b * s->ldx));
   SHIP(s, s->S0.ensure((size_t)b));
   SHIP(s, s->loss_part.ensure((size_t)(b + 255) / 256));
   s->cap = b;
   return FDT_OK;
 }
 
-static GemmArgs gemm(int M, int N, int K, const uint16_t* A, long sam, long sak, const uint16_t* B, long sbk, long sbn) {
+static GemmOperand operand(const uint16_t* p, long ld, bool kc) {
+  GemmOperand o{};
+  o.p = p; o.ld = ld; o.kc = kc;
+  o.vec = ld % 8 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+  return o;
+}
+static GemmArgs gemm(int M, int N, int K, GemmOperand a, GemmOperand b) {
   GemmArgs g{};
   g.M = M; g.N = N; g.K = K;
-  g.A = A; g.sam = sam; g.sak = sak;
-  g.B = B; g.sbk = sbk; g.sbn = sbn;
+  g.a = a; g.b = b;
   g.ldc = N;
   return g;
 }
 
-// forward of b rows of X (bf16 [b][n_in]); keeps Z (pre-activations) when
+// forward of b rows of X (bf16 [b][ldx]); keeps Z (pre-activations) when
 // `keep`, the output in Z[3]
 static int sg_forward(fdt_surrogate* s, const uint16_t* X, int b, bool keep) {
   const uint16_t* in = X;
   for (int l = 0; l < SG_LAYERS; ++l) {
     const int K = s->dims[l], N = s->dims[l + 1];
-    GemmArgs g = gemm(b, N, K, in, K, 1, s->wb.p + s->woff[l], N, 1);
+    GemmArgs g = gemm(b, N, K, operand(in, l ? K : s->ldx, true), operand(s->wb.p + s->woff[l], N, false));
     g.bias = s->w.p + s->boff[l];
     const bool last = l == SG_LAYERS - 1;
     g.C = (keep || last) ? s->Z[l].p : nullptr;
     g.Cb = last ? nullptr : s->A[l].p;
-    g.act = last ? 0 : 1;
+    g.act = last ? GEMM_LINEAR : GEMM_GELU;
     SHIP(s, fdt_launch_gemm_bf16(&g, s->stream));
     in = s->A[l].p;
   }
@@ -1562,21 +1565,26 @@ static int sg_forward(fdt_surrogate* s, const uint16_t* X, int b, bool keep) {
 // gradients of the mean loss over b rows into s->g; loss sum into *loss (host)
 static int sg_backward(fdt_surrogate* s, const uint16_t* X, const float* T, int b, float* loss) {
   const int nb = (b + 255) / 256;
-  SHIP(s, fdt_launch_sg_loss(s->Z[SG_LAYERS - 1].p, T, b, s->dZ.p, s->loss_part.p, 0.1f, s->stream));
+  uint16_t* dZ = s->dZ[0].p;  // of layer l; the layer below gets the other buffer
+  SHIP(s, fdt_launch_sg_loss(s->Z[SG_LAYERS - 1].p, T, b, dZ, s->loss_part.p, 0.1f, s->stream));
   for (int l = SG_LAYERS - 1; l >= 0; --l) {
     const int K = s->dims[l], N = s->dims[l + 1];
-    const uint16_t* in = l ? s->A[l - 1].p : X;
-    // dW = in^T . dZ  (K x N, reduced over the batch)
-    GemmArgs gw = gemm(K, N, b, in, 1, K, s->dZ.p, N, 1);
+    const long ldz = l == SG_LAYERS - 1 ? SG_LDO : N;
+    // dW = in^T . dZ  (K x N, reduced over the batch); its row K is db, the
+    // column sums of dZ, which follow dW in the flat gradients
+    GemmArgs gw = gemm(K, N, b, operand(l ? s->A[l - 1].p : X, l ? K : s->ldx, false), operand(dZ, ldz, false));
+    gw.a.ones = true;
     gw.C = s->g.p + s->woff[l];
     SHIP(s, fdt_launch_gemm_bf16(&gw, s->stream));
-    SHIP(s, fdt_launch_mlp_ew(1, s->dZ.p, nullptr, s->g.p + s->boff[l], 0, b, N, s->stream));
     if (l == 0) break;
-    // dA = dZ . W^T  (b x K), then dZ = dA * gelu'(Z[l-1])
-    GemmArgs ga = gemm(b, K, N, s->dZ.p, N, 1, s->wb.p + s->woff[l], 1, N);
-    ga.C = s->dA.p;
+    // dZ of the layer below = (dZ . W^T) * gelu'(Z[l-1])  (b x K)
+    uint16_t* below = dZ == s->dZ[0].p ? s->dZ[1].p : s->dZ[0].p;
+    GemmArgs ga = gemm(b, K, N, operand(dZ, ldz, true), operand(s->wb.p + s->woff[l], N, true));
+    ga.Cb = below;
+    ga.act = GEMM_GELU_BWD;
+    ga.Z = s->Z[l - 1].p;
     SHIP(s, fdt_launch_gemm_bf16(&ga, s->stream));
-    SHIP(s, fdt_launch_mlp_ew(0, s->dA.p, s->Z[l - 1].p, s->dZ.p, (size_t)b * K, 0, 0, s->stream));
+    dZ = below;
   }
   if (loss) {
     std::vector<float> part(nb);
@@ -1596,6 +1604,7 @@ fdt_surrogate* fdt_surrogate_create(int device, int n_in, uint64_t seed) {
   fdt_surrogate* s = new fdt_surrogate;
   s->device = device;
   s->n_in = n_in;
+  s->ldx = (n_in + 7) / 8 * 8;
   const int d[SG_LAYERS + 1] = {n_in, SG_HID0, SG_HID1, SG_HID2, SG_OUT};
   size_t off = 0;
   for (int l = 0; l <= SG_LAYERS; ++l) s->dims[l] = d[l];
@@ -1629,9 +1638,10 @@ void fdt_surrogate_destroy(fdt_surrogate* s) {
   if (!s) return;
   (void)hipSetDevice(s->device);
   if (s->stream) (void)hipStreamSynchronize(s->stream);
-  DevBuf<float>* fb[] = {&s->w, &s->m, &s->v, &s->g, &s->T, &s->bvals, &s->dA, &s->loss_part, &s->S0};
+  DevBuf<float>* fb[] = {&s->w, &s->m, &s->v, &s->g, &s->T, &s->bvals, &s->loss_part, &s->S0};
   for (auto* b : fb) b->release();
-  s->wb.release(); s->X.release(); s->dZ.release(); s->Xb.release();
+  s->wb.release(); s->X.release(); s->Xb.release();
+  for (auto& d : s->dZ) d.release();
   for (int l = 0; l < SG_LAYERS; ++l) { s->Z[l].release(); s->A[l].release(); }
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
@@ -1646,7 +1656,7 @@ int fdt_surrogate_load(fdt_surrogate* s, const float* w, size_t n) {
   if (n != s->nw) return serr(s, FDT_EINVAL, "%zu weights given, the network has %zu", n, s->nw);
   (void)hipSetDevice(s->device);
   SHIP(s, hipMemcpyAsync(s->w.p, w, sizeof(float) * n, hipMemcpyHostToDevice, s->stream));
-  SHIP(s, fdt_launch_mlp_ew(2, s->w.p, nullptr, s->wb.p, n, 0, 0, s->stream));
+  SHIP(s, fdt_launch_to_bf16(s->w.p, s->wb.p, n, s->stream));
   SHIP(s, hipMemsetAsync(s->m.p, 0, sizeof(float) * n, s->stream));
   SHIP(s, hipMemsetAsync(s->v.p, 0, sizeof(float) * n, s->stream));
   SHIP(s, hipStreamSynchronize(s->stream));
@@ -1671,12 +1681,12 @@ int fdt_surrogate_set_training_data(fdt_surrogate* s, const float* signals, cons
   DevBuf<float> raw;
   SHIP(s, raw.ensure((size_t)n * N));
   SHIP(s, s->bvals.ensure(N));
-  SHIP(s, s->X.ensure((size_t)n * N));
+  SHIP(s, s->X.ensure((size_t)n * s->ldx));
   SHIP(s, s->T.ensure((size_t)n * SG_OUT));
   SHIP(s, hipMemcpyAsync(raw.p, signals, sizeof(float) * n * N, hipMemcpyHostToDevice, s->stream));
   SHIP(s, hipMemcpyAsync(s->bvals.p, bvals, sizeof(float) * N, hipMemcpyHostToDevice, s->stream));
   SHIP(s, hipMemcpyAsync(s->T.p, targets, sizeof(float) * n * SG_OUT, hipMemcpyHostToDevice, s->stream));
-  SHIP(s, fdt_launch_normalize(raw.p, N, n, s->bvals.p, 50.0f, s->X.p, nullptr, s->stream));
+  SHIP(s, fdt_launch_normalize(raw.p, N, n, s->bvals.p, 50.0f, s->X.p, s->ldx, nullptr, s->stream));
   SHIP(s, hipStreamSynchronize(s->stream));
   raw.release();
   s->ntrain = n;
@@ -1688,7 +1698,7 @@ int fdt_surrogate_gradients(fdt_surrogate* s, int first, int batch, float* grads
   if (!s || batch <= 0 || first < 0 || first + batch > s->ntrain) return serr(s, FDT_EINVAL, "bad batch");
   (void)hipSetDevice(s->device);
   if (int rc = sg_reserve(s, batch)) return rc;
-  const uint16_t* X = s->X.p + (size_t)first * s->n_in;
+  const uint16_t* X = s->X.p + (size_t)first * s->ldx;
   if (int rc = sg_forward(s, X, batch, true)) return rc;
   if (int rc = sg_backward(s, X, s->T.p + (size_t)first * SG_OUT, batch, loss)) return rc;
   if (grads) {
@@ -1721,7 +1731,7 @@ int fdt_surrogate_forward(fdt_surrogate* s, const float* signals, const float* b
   if (int rc = sg_reserve(s, std::min(n, chunk))) return rc;
   for (int c0 = 0; c0 < n; c0 += chunk) {
     const int b = std::min(chunk, n - c0);
-    SHIP(s, fdt_launch_normalize(raw.p + (size_t)c0 * N, N, b, s->bvals.p, 50.0f, s->Xb.p, nullptr, s->stream));
+    SHIP(s, fdt_launch_normalize(raw.p + (size_t)c0 * N, N, b, s->bvals.p, 50.0f, s->Xb.p, s->ldx, nullptr, s->stream));
     if (int rc = sg_forward(s, s->Xb.p, b, false)) return rc;
     SHIP(s, hipMemcpyAsync(out + (size_t)c0 * SG_OUT, s->Z[SG_LAYERS - 1].p, sizeof(float) * b * SG_OUT,
                            hipMemcpyDeviceToHost, s->stream));
@@ -1747,7 +1757,7 @@ static int sg_infer(fdt_surrogate* s, fdt_ctx* c, DevBuf<float>& dir) {
   if (int rc = sg_reserve(s, std::min(std::max(nv, 1), chunk))) return rc;
   for (int c0 = 0; c0 < nv; c0 += chunk) {
     const int b = std::min(chunk, nv - c0);
-    SHIP(s, fdt_launch_normalize(c->d_data.p + (size_t)c0 * c->N, c->N, b, c->d_bvals.p, 50.0f, s->Xb.p, s->S0.p,
+    SHIP(s, fdt_launch_normalize(c->d_data.p + (size_t)c0 * c->N, c->N, b, c->d_bvals.p, 50.0f, s->Xb.p, s->ldx, s->S0.p,
                                  c->stream));
     // the network runs on the context's stream
     hipStream_t keep = s->stream;

@@ -9,22 +9,30 @@ constexpr int SG_OUT = 28;     // 3 f + 3x3 directions + d + d_std + 14 log prop
 constexpr int SG_LAYERS = 4;   // N -> 512 -> 512 -> 256 -> 28
 constexpr int SG_HID0 = 512, SG_HID1 = 512, SG_HID2 = 256;
 
-// C[m][n] (row-major, leading dimension ldc) = sum_k A(m,k) B(k,n) with
-// A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn] (bf16 storage);
-// epilogue: (+ C if accumulate) (+ bias[n]) -> C (fp32, optional) and
-// act ? gelu : identity -> Cb (bf16, optional, same indexing)
+constexpr int SG_LDO = 32;     // row length of the output gradients (zero padded)
+
+// An operand of the GEMM, bf16, rows along m (A) or n (B): element (row, k) at
+// p[row * ld + k] (kc) or p[k * ld + row]; vec: p and ld are 16-byte multiples.
+// ones (A, not kc): row M of A is all ones, so that row M of C is the column
+// sum of B
+struct GemmOperand {
+  const uint16_t* p;
+  long ld;
+  bool kc, vec, ones;
+};
+enum { GEMM_LINEAR = 0, GEMM_GELU = 1, GEMM_GELU_BWD = 2 };
+// C[m][n] (row-major, leading dimension ldc) = sum_k A(m,k) B(n,k) (+ bias[n])
+// -> C (fp32, optional) and act of it -> Cb (bf16, optional, same indexing);
+// GEMM_GELU_BWD: C gelu'(Z)
 struct GemmArgs {
   int M, N, K;
-  const uint16_t* A;
-  long sam, sak;
-  const uint16_t* B;
-  long sbk, sbn;
+  GemmOperand a, b;
   float* C;
   uint16_t* Cb;
   long ldc;
   const float* bias;
   int act;
-  int accumulate;
+  const float* Z;
 };
 
 struct SgDecodeArgs {

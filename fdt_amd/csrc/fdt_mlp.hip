@@ -4,12 +4,9 @@
 // normalisation, decoding of the network outputs into chain start values and
 // proposal widths, the fallback test).
 //
-// GEMM: C[M x N] = A[M x K] . B[K x N] with arbitrary element strides for A
-// and B (so X.W, dZ.W^T and X^T.dZ are one kernel).  A 256-thread workgroup
-// computes a 64x64 tile; each wave a 32x32 quadrant as 2x2 blocks of
-// v_mfma_f32_16x16x32_bf16 (FP32 accumulation), K in steps of 32 staged in
-// LDS (A row-major, B column-major so that every lane's 8 K values are one
-// 16-byte LDS read).
+// GEMM: C[M x N] = A[M x K] . B[K x N] in v_mfma_f32_16x16x32_bf16 (FP32
+// accumulation).  Each operand is stored with k contiguous or with m (n)
+// contiguous, so X.W, dZ.W^T and X^T.dZ are one kernel.
 #include "fdt_device.h"
 #include "fdt_mlp.h"
 
@@ -30,84 +27,154 @@ FDT_DEV float gelu_grad(float x) {
   return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
 }
 
-constexpr int GT = 64;   // tile edge
-constexpr int GK = 32;   // K step
-constexpr int GLD = 40;  // LDS row stride in bf16 (80 bytes)
+// A 256-thread workgroup computes a TM x TN tile, each of its 2 x 2 waves a
+// quadrant in 16 x 16 blocks, K in steps of 64.  What bounds it: the forward
+// of 65,536 rows is memory- and LDS-fed MFMA work (128 x 128 tiles reuse every
+// staged element 128 times; 64 x 64 tiles with 2-byte loads, as before, ran
+// 50 TFLOP/s), a training step's products are a few hundred thousand outputs
+// and bound by latency, so their tiles shrink until every CU has one.  The
+// next step's global loads (16 bytes a lane) are in flight while a step
+// multiplies; LDS rows are 144 bytes, which spreads a wave's 16-byte reads
+// over all banks.  An operand with m (n) contiguous is transposed on its way
+// to LDS in pairs of k.  Every output is the same chain of 32-wide products
+// in k order for every tile.
+constexpr int GK = 64;   // K step
+constexpr int GLD = 72;  // LDS row stride in bf16
 
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[GT * GLD];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[GT * GLD];  // [n][k]
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
-  const int qm = (wave >> 1) * 32, qn = (wave & 1) * 32;
-  f32x4 acc[2][2];
+typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+
+// one operand's tile of T rows (m or n) by GK: fetched to registers, then stored to LDS [row][k]
+template <int T, bool KC>
+struct Stage {
+  static constexpr int UNITS = T * GK / 8;  // of 8 elements
+  static constexpr int NU = KC || UNITS >= 512 ? UNITS / 256 : 2;  // per thread
+  static_assert(KC ? UNITS >= 256 : UNITS >= 256 && T % 32 == 0, "tile too small");
+  // a tile of 32 rows has pairs for half of the threads only
+  static FDT_DEV bool mine() { return KC || UNITS >= 512 || threadIdx.x < UNITS / 2; }
+  u16x8 v[NU];
+  // unit u: KC: row u / 8, k (u % 8) * 8.  Otherwise units come in pairs (k, k + 1) of 8 rows: four 8-row groups
+  // and 16 k pairs per wave (64-byte runs of global memory, two lanes per LDS bank)
+  static FDT_DEV void where(int i, int& row, int& k) {
+    const int t = threadIdx.x;
+    if constexpr (KC) {
+      const int u = t + 256 * i;
+      row = u >> 3;
+      k = (u & 7) * 8;
+    } else {
+      const int p = t + 256 * (i >> 1);  // T / 8 * GK / 2 pairs
+      const int g = p >> 6;              // wave-sized block: T / 32 row blocks, then two k halves
+      row = ((g % (T / 32)) * 4 + (p & 3)) * 8;
+      k = ((g / (T / 32)) * 16 + ((p >> 2) & 15)) * 2 + (i & 1);
+    }
+  }
+  FDT_DEV void fetch(const GemmOperand& o, int row0, int rows, int k0, int K) {
+    if (!mine()) return;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NU; ++i) {
+      int r, k;
+      where(i, r, k);
+      r += row0;
+      k += k0;
+      const uint16_t* p = o.p + (KC ? (size_t)r * o.ld + k : (size_t)k * o.ld + r);
+      const bool whole = KC ? (r < rows && k + 8 <= K) : (k < K && r + 8 <= rows);
+      if (whole && o.vec) v[i] = *reinterpret_cast<const u16x8*>(p);
+      else {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  // staging: thread t fills row (t / 4) of the tile, K elements (t % 4) * 8 .. + 8
-  const int sr = tid >> 2, sk = (tid & 3) * 8;
-  for (int k0 = 0; k0 < g.K; k0 += GK) {
-    {
-      const int m = m0 + sr;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int k = k0 + sk + e;
-        As[sr * GLD + sk + e] = (m < g.M && k < g.K) ? g.A[(size_t)m * g.sam + (size_t)k * g.sak] : (uint16_t)0;
-      }
-      const int n = n0 + sr;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int k = k0 + sk + e;
-        Bs[sr * GLD + sk + e] = (n < g.N && k < g.K) ? g.B[(size_t)k * g.sbk + (size_t)n * g.sbn] : (uint16_t)0;
+        for (int e = 0; e < 8; ++e) {
+          const int re = KC ? r : r + e, ke = KC ? k + e : k;
+          uint16_t x = 0;
+          if (ke < K) {
+            if (re < rows) x = p[e];
+            else if (re == rows && o.ones) x = 0x3F80;  // bf16 1
+          }
+          v[i][e] = x;
+        }
       }
     }
+  }
+  FDT_DEV void store(uint16_t* lds) const {
+    if (!mine()) return;
+#pragma unroll
+    for (int i = 0; i < NU; i += KC ? 1 : 2) {
+      int r, k;
+      where(i, r, k);
+      if constexpr (KC) *reinterpret_cast<u16x8*>(&lds[r * GLD + k]) = v[i];
+      else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          *reinterpret_cast<uint32_t*>(&lds[(r + e) * GLD + k]) = (uint32_t)v[i][e] | ((uint32_t)v[i + 1][e] << 16);
+      }
+    }
+  }
+};
+
+template <int TM, int TN, bool AK, bool BK>
+__global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) uint16_t As[TM * GLD];
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[TN * GLD];  // [n][k]
+  constexpr int MB = TM / 32, NB = TN / 32;                       // 16 x 16 blocks of a wave's quadrant
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int rows = g.M + (g.a.ones ? 1 : 0);
+  // The n tiles of one m tile follow each other on one XCD (workgroups go
+  // round robin over the 8), so that its L2 holds the A rows they share
+  const int nt = (g.N + TN - 1) / TN, mt = (rows + TM - 1) / TM;
+  int b = blockIdx.x, tm, tn;
+  if (b < (mt >> 3) * 8 * nt) { tm = (b >> 3) / nt * 8 + (b & 7); tn = (b >> 3) % nt; }
+  else { tm = b / nt; tn = b % nt; }
+  const int m0 = tm * TM, n0 = tn * TN;
+  const int qm = (wave >> 1) * (TM / 2), qn = (wave & 1) * (TN / 2);
+  f32x4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  Stage<TM, AK> sa;
+  Stage<TN, BK> sb;
+  sa.fetch(g.a, m0, g.M, 0, g.K);
+  sb.fetch(g.b, n0, g.N, 0, g.K);
+  const int r = lane & 15, kb = (lane >> 4) * 8;
+  for (int k0 = 0; k0 < g.K; k0 += GK) {
+    sa.store(As);
+    sb.store(Bs);
     __syncthreads();
-    const int r = lane & 15, kb = (lane >> 4) * 8;
-    bf16x8 a[2], b[2];
+    if (k0 + GK < g.K) {
+      sa.fetch(g.a, m0, g.M, k0 + GK, g.K);
+      sb.fetch(g.b, n0, g.N, k0 + GK, g.K);
+    }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const bf16x8*>(&As[(qm + 16 * i + r) * GLD + kb]);
+    for (int h = 0; h < GK; h += 32) {
+      if (k0 + h >= g.K) break;
+      bf16x8 a[MB], bb[NB];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const bf16x8*>(&Bs[(qn + 16 * j + r) * GLD + kb]);
+      for (int i = 0; i < MB; ++i) a[i] = *reinterpret_cast<const bf16x8*>(&As[(qm + 16 * i + r) * GLD + h + kb]);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+      for (int j = 0; j < NB; ++j) bb[j] = *reinterpret_cast<const bf16x8*>(&Bs[(qn + 16 * j + r) * GLD + h + kb]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bb[j], acc[i][j], 0, 0, 0);
+    }
     __syncthreads();
   }
   // lane holds C[(lane / 16) * 4 + v][lane % 16] of each 16x16 block
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int j = 0; j < NB; ++j) {
+    const int n = n0 + qn + 16 * j + (lane & 15);
+    if (n >= g.N) continue;
+    const float bias = g.bias ? g.bias[n] : 0.0f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int m = m0 + qm + 16 * i + (lane >> 4) * 4 + v;
-        const int n = n0 + qn + 16 * j + (lane & 15);
-        if (m >= g.M || n >= g.N) continue;
+        if (m >= rows) continue;
         float x = acc[i][j][v];
         const size_t ci = (size_t)m * g.ldc + n;
-        if (g.accumulate) x += g.C[ci];
-        if (g.bias) x += g.bias[n];
+        if (g.bias) x += bias;
         if (g.C) g.C[ci] = x;
-        if (g.Cb) g.Cb[ci] = f2bf(g.act ? gelu(x) : x);
+        if (g.Cb) g.Cb[ci] = f2bf(g.act == GEMM_GELU ? gelu(x) : g.act == GEMM_GELU_BWD ? x * gelu_grad(g.Z[ci]) : x);
       }
-}
-
-// dZ (bf16) = dA * gelu'(Z)
-__global__ void gelu_bwd_kernel(const float* dA, const float* Z, uint16_t* dZ, size_t n) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dZ[i] = f2bf(dA[i] * gelu_grad(Z[i]));
-}
-
-// db[n] = sum_m dZ[m][n] (dZ bf16, M x N), one thread per column, fixed order
-__global__ void colsum_kernel(const uint16_t* dZ, int M, int N, float* db) {
-  int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.0f;
-  for (int m = 0; m < M; ++m) s += bf2f(dZ[(size_t)m * N + n]);
-  db[n] = s;
+  }
 }
 
 // Adam (Kingma & Ba 2015) on FP32 master weights, with a BF16 copy for the GEMMs
@@ -131,25 +198,29 @@ __global__ void to_bf16_kernel(const float* x, uint16_t* y, size_t n) {
 }
 
 // Network input: the voxel's signal over the mean of its b=0 volumes (the
-// volumes with b <= b0_max), one thread per voxel
-__global__ void normalize_kernel(const float* data, int N, int nvox, const float* bvals, float b0_max, uint16_t* X,
-                                 float* S0) {
-  int v = blockIdx.x * blockDim.x + threadIdx.x;
+// volumes with b <= b0_max), one 16-lane row per voxel; rows of X are ldx long,
+// zero beyond N.  Bound by the read of the signals (one thread per voxel read
+// them in 4-byte strides: 170 us per 65,536 voxels of 288 volumes).
+__global__ __launch_bounds__(256) void normalize_kernel(const float* data, int N, int nvox, const float* bvals,
+                                                        float b0_max, uint16_t* X, int ldx, float* S0) {
+  const int v = blockIdx.x * 16 + (threadIdx.x >> 4), rl = threadIdx.x & 15;
   if (v >= nvox) return;
   const float* y = data + (size_t)v * N;
   double s = 0.0;
   int nb = 0;
-  for (int i = 0; i < N; ++i)
+  for (int i = rl; i < N; i += 16)
     if (bvals[i] <= b0_max) { s += y[i]; ++nb; }
+  s = row_sum16_d(s);
+  nb = (int)row_sum16((float)nb);
   float s0 = nb ? (float)(s / nb) : 1.0f;
   if (!(s0 > 0.0f)) s0 = 1.0f;
   float inv = 1.0f / s0;
-  for (int i = 0; i < N; ++i) X[(size_t)v * N + i] = f2bf(y[i] * inv);
-  if (S0) S0[v] = s0;
+  for (int i = rl; i < ldx; i += 16) X[(size_t)v * ldx + i] = i < N ? f2bf(y[i] * inv) : (uint16_t)0;
+  if (S0 && rl == 0) S0[v] = s0;
 }
 
 // Loss on the network outputs O [M][SG_OUT] against targets T [M][SG_OUT] and
-// its gradient dO (bf16, the last layer has no activation).  Targets: f_k (3),
+// its gradient dO (bf16 [M][SG_LDO], zero padded; the last layer has no activation).  Targets: f_k (3),
 // dyads x_k (3 x 3, sign-free: loss |p|^4 - 2 (p.x)^2 + 1 = ||p p^T - x x^T||^2
 // weighted by f_k), 1000 d, 1000 d_std, log proposal widths (weight w_lw,
 // zero where the target slot is unused, marked by a target >= 1e29).
@@ -159,8 +230,8 @@ __global__ void sg_loss_kernel(const float* O, const float* T, int M, uint16_t* 
   if (m < M) {
     const float* o = O + (size_t)m * SG_OUT;
     const float* t = T + (size_t)m * SG_OUT;
-    float g[SG_OUT];
-    for (int i = 0; i < SG_OUT; ++i) g[i] = 0.0f;
+    float g[SG_LDO];
+    for (int i = 0; i < SG_LDO; ++i) g[i] = 0.0f;
     for (int k = 0; k < 3; ++k) {
       float e = o[k] - t[k];
       l += e * e;
@@ -186,7 +257,7 @@ __global__ void sg_loss_kernel(const float* O, const float* T, int M, uint16_t* 
       l += w_lw * e * e;
       g[i] = 2.0f * w_lw * e;
     }
-    for (int i = 0; i < SG_OUT; ++i) dO[(size_t)m * SG_OUT + i] = f2bf(g[i] / (float)M);
+    for (int i = 0; i < SG_LDO; ++i) dO[(size_t)m * SG_LDO + i] = i < SG_OUT ? f2bf(g[i] / (float)M) : (uint16_t)0;
   }
   // block partial sums of the loss (fixed order within the block)
   __shared__ float red[256];
@@ -274,22 +345,33 @@ __global__ void sg_fallback_kernel(SgFallbackArgs a) {
 
 }  // namespace fdt
 
-extern "C" hipError_t fdt_launch_gemm_bf16(const fdt::GemmArgs* g, hipStream_t s) {
-  if (g->M <= 0 || g->N <= 0) return hipSuccess;
-  dim3 grid((g->N + fdt::GT - 1) / fdt::GT, (g->M + fdt::GT - 1) / fdt::GT), block(256);
-  hipLaunchKernelGGL(fdt::gemm_bf16_kernel, grid, block, 0, s, *g);
+namespace {
+template <int TM, int TN>
+hipError_t launch_tile(const fdt::GemmArgs* g, hipStream_t s) {
+  const int rows = g->M + (g->a.ones ? 1 : 0);
+  const dim3 grid((unsigned)(((rows + TM - 1) / TM) * ((g->N + TN - 1) / TN))), block(256);
+  if (g->a.kc && g->b.kc) hipLaunchKernelGGL((fdt::gemm_bf16_kernel<TM, TN, true, true>), grid, block, 0, s, *g);
+  else if (g->a.kc) hipLaunchKernelGGL((fdt::gemm_bf16_kernel<TM, TN, true, false>), grid, block, 0, s, *g);
+  else if (!g->b.kc) hipLaunchKernelGGL((fdt::gemm_bf16_kernel<TM, TN, false, false>), grid, block, 0, s, *g);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
+}  // namespace
 
-extern "C" hipError_t fdt_launch_mlp_ew(int op, const void* a, const void* b, void* c, size_t n, int M, int N,
-                                        hipStream_t s) {
-  dim3 block(256), grid((unsigned)((n + 255) / 256));
-  switch (op) {
-    case 0: hipLaunchKernelGGL(fdt::gelu_bwd_kernel, grid, block, 0, s, (const float*)a, (const float*)b, (uint16_t*)c, n); break;
-    case 1: hipLaunchKernelGGL(fdt::colsum_kernel, dim3((N + 255) / 256), block, 0, s, (const uint16_t*)a, M, N, (float*)c); break;
-    case 2: hipLaunchKernelGGL(fdt::to_bf16_kernel, grid, block, 0, s, (const float*)a, (uint16_t*)c, n); break;
-    default: return hipErrorInvalidValue;
-  }
+// The largest tile that still gives each of the 256 CUs a workgroup; outputs
+// of at most 32 columns do not fill wider tiles
+extern "C" hipError_t fdt_launch_gemm_bf16(const fdt::GemmArgs* g, hipStream_t s) {
+  if (g->M <= 0 || g->N <= 0) return hipSuccess;
+  const int rows = g->M + (g->a.ones ? 1 : 0);
+  auto tiles = [&](int tm, int tn) { return (long)((rows + tm - 1) / tm) * ((g->N + tn - 1) / tn); };
+  if (g->N <= 32) return tiles(128, 32) >= 256 ? launch_tile<128, 32>(g, s) : launch_tile<32, 32>(g, s);
+  if (tiles(128, 128) >= 256) return launch_tile<128, 128>(g, s);
+  if (tiles(64, 64) >= 256) return launch_tile<64, 64>(g, s);
+  return launch_tile<32, 32>(g, s);
+}
+
+extern "C" hipError_t fdt_launch_to_bf16(const float* x, uint16_t* y, size_t n, hipStream_t s) {
+  hipLaunchKernelGGL(fdt::to_bf16_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, y, n);
   return hipGetLastError();
 }
 
@@ -302,9 +384,10 @@ extern "C" hipError_t fdt_launch_adam(float* w, float* m, float* v, const float*
 }
 
 extern "C" hipError_t fdt_launch_normalize(const float* data, int N, int nvox, const float* bvals, float b0_max,
-                                           uint16_t* X, float* S0, hipStream_t s) {
+                                           uint16_t* X, int ldx, float* S0, hipStream_t s) {
   if (nvox <= 0) return hipSuccess;
-  hipLaunchKernelGGL(fdt::normalize_kernel, dim3((nvox + 255) / 256), dim3(256), 0, s, data, N, nvox, bvals, b0_max, X, S0);
+  hipLaunchKernelGGL(fdt::normalize_kernel, dim3((nvox + 15) / 16), dim3(256), 0, s, data, N, nvox, bvals, b0_max, X, ldx,
+                     S0);
   return hipGetLastError();
 }
 
