@@ -58,9 +58,12 @@ hipError_t fdt_launch_grad_acq(const float4* base, int N, int stride, const floa
 #define FDT_VPL_DECL(V) hipError_t fdt_launch_mcmc_vpl##V(const McmcArgs*, int, int, hipStream_t);
 FDT_VPL_DECL(3)
 FDT_VPL_DECL(5)
+FDT_VPL_DECL(7)
 FDT_VPL_DECL(10)
+FDT_VPL_DECL(14)
 FDT_VPL_DECL(18)
 FDT_VPL_DECL(24)
+FDT_VPL_DECL(27)
 FDT_VPL_DECL(32)
 }
 
@@ -68,13 +71,24 @@ namespace {
 
 typedef hipError_t (*mcmc_launch_fn)(const McmcArgs*, int, int, hipStream_t);
 struct VplEntry { int vpl; mcmc_launch_fn fn; };
-const VplEntry kVpl[] = {{3, fdt_launch_mcmc_vpl3}, {5, fdt_launch_mcmc_vpl5}, {10, fdt_launch_mcmc_vpl10},
-                         {18, fdt_launch_mcmc_vpl18}, {24, fdt_launch_mcmc_vpl24}, {32, fdt_launch_mcmc_vpl32}};
+// In steps of about a third, so that little of a tile is padding: with 3, 5, 10, 18, 24 and 32 alone the chains of
+// 432 volumes ran in 32 slots instead of 27 (3,001 voxels, model 2, K = 2, --f0: 68.0 -> 61.0 ms with the fit), those
+// of 200 volumes in 18 instead of 14
+const VplEntry kVpl[] = {{3, fdt_launch_mcmc_vpl3},   {5, fdt_launch_mcmc_vpl5},   {7, fdt_launch_mcmc_vpl7},
+                         {10, fdt_launch_mcmc_vpl10}, {14, fdt_launch_mcmc_vpl14}, {18, fdt_launch_mcmc_vpl18},
+                         {24, fdt_launch_mcmc_vpl24}, {27, fdt_launch_mcmc_vpl27}, {32, fdt_launch_mcmc_vpl32}};
 
 // the MCMC tile (volumes per lane) for N volumes, at least `force`
 int tile_of(int N, int force) {
   for (const auto& e : kVpl)
     if (16 * e.vpl >= N && e.vpl >= force) return e.vpl;
+  return 0;
+}
+
+// the tile of a volume in the queue kernel, which carries four of them
+int queue_tile_of(int N, int force) {
+  for (int vpl : {3, 5, 10, 18})
+    if (16 * vpl >= N && vpl >= force) return vpl;
   return 0;
 }
 
@@ -1180,8 +1194,7 @@ static void queue_invalidate(fdt_queue* q) {
 // jobs the queue kernel carries; Rician, --gradnonlin and the widest tiles run
 // their own chain launch inside the batch
 static bool in_queue_kernel(const fdt_ctx* c) {
-  int vpl = tile_of(c->N, c->vpl_force);
-  return !c->o.rician && !c->gn && vpl > 0 && vpl <= QUEUE_MAX_VPL;
+  return !c->o.rician && !c->gn && queue_tile_of(c->N, c->vpl_force) > 0;
 }
 
 static int queue_launch_chains(fdt_queue* q, const QueueJob* d_jobs, int njobs, const int* d_first, int total) {
@@ -1220,7 +1233,7 @@ static int queue_issue(fdt_queue* q, bool upload) {
       mcmc_launch_fn fn = nullptr;
       QCTX(q, c, mcmc_prepare(c, c->vox_offset, &j.a, &fn));
       j.K = c->o.nfibres;
-      j.vpl = c->vpl_used;
+      j.vpl = queue_tile_of(c->N, c->vpl_force);
       q->h_jobs.push_back(j);
       q->h_first.push_back(q->h_first.back() + (c->nvox + q->rows_per_wg - 1) / q->rows_per_wg);
     }
@@ -1386,7 +1399,10 @@ int fdt_queue_timing(fdt_queue* q, float* ms_last, int* rows_per_wg, int* vpl_of
   if (ms_last) *ms_last = q->ms_last;
   if (rows_per_wg) *rows_per_wg = q->rows_per_wg;
   if (vpl_of_job)
-    for (int j = 0; j < njobs && j < (int)q->jobs.size(); ++j) vpl_of_job[j] = tile_of(q->jobs[j]->N, q->jobs[j]->vpl_force);
+    for (int j = 0; j < njobs && j < (int)q->jobs.size(); ++j) {
+      const fdt_ctx* c = q->jobs[j];
+      vpl_of_job[j] = in_queue_kernel(c) ? queue_tile_of(c->N, c->vpl_force) : tile_of(c->N, c->vpl_force);
+    }
   return FDT_OK;
 }
 
@@ -1415,7 +1431,7 @@ int fdt_queue_autotune(fdt_queue* q, int jumps, int sample_vox, float* ms_best) 
       mcmc_launch_fn fn = nullptr;
       QCTX(q, c, mcmc_prepare(c, c->vox_offset, &j.a, &fn));
       j.K = c->o.nfibres;
-      j.vpl = c->vpl_used;
+      j.vpl = queue_tile_of(c->N, c->vpl_force);
       j.a.nvox = std::min(c->nvox, sample_vox);
       j.a.nburn = 0;
       j.a.njumps = jumps;
@@ -1456,9 +1472,9 @@ int fdt_queue_autotune(fdt_queue* q, int jumps, int sample_vox, float* ms_best) 
   q->rows_per_wg = best_rows;
   for (fdt_ctx* c : q->jobs) {
     if (!in_queue_kernel(c)) continue;
-    int cur = tile_of(c->N, c->vpl_force);
-    int next = tile_of(c->N, cur + 1);
-    if (!next || next > QUEUE_MAX_VPL) continue;
+    int cur = queue_tile_of(c->N, c->vpl_force);
+    int next = queue_tile_of(c->N, cur + 1);
+    if (!next) continue;
     int keep = c->vpl_force;
     c->vpl_force = next;
     float ms;

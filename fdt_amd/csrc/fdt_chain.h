@@ -65,12 +65,12 @@ FDT_DEV void sincos_full(float x, float& s, float& c) {
 enum { SL_F0 = 0, SL_TAU = 1, SL_D = 2, SL_DSTD = 3, SL_R = 4, SL_S0 = 5, SL_FIB = 6 };
 
 // Tiles whose chains stage b = 0 volumes first and skip their slot (see
-// stage_acq): the 18-volume tile, where it saves 3-4% of the chain time.  In
+// stage_acq): the 14- and 18-volume tiles, where it saves 3-4% of the chain time.  In
 // the smaller tiles the uniform branch around slot 0 costs more than it saves
 // (it splits the few volumes a lane interleaves); at 24 and 32 volumes per
 // lane (one wave per SIMD) it saved nothing (N = 384 with 24 b = 0 volumes)
 // and cost 1.4% (N = 432).
-template <int VPL> constexpr bool ZERO_SLOT = VPL == 18;
+template <int VPL> constexpr bool ZERO_SLOT = VPL == 14 || VPL == 18;
 
 // Signal forms with row-uniform coefficients (compute_signal /
 // compute_iso_signal, CUDA/runmcmc_kernels.cu:67-95):
@@ -176,8 +176,11 @@ struct Quad {
 // per proposal) instead of letting the loop-invariant loads be hoisted into
 // ~4*VPL VGPRs for the whole chain.
 FDT_DEV void reload_acq() { asm volatile("" ::: "memory"); }
-FDT_DEV int acc1(int c) { return c + 1; }
-FDT_DEV int rej1(int c) { return c + (1 << 16); }
+// x^2 rounded on its own: not contracted into a sum, with padding masks or without
+FDT_DEV float square(float x) {
+#pragma clang fp contract(off)
+  return x * x;
+}
 
 
 // One chain per 16-lane row.  Volume state lives in registers per lane;
@@ -191,7 +194,7 @@ FDT_DEV int rej1(int c) { return c + (1 << 16); }
 // the stick signals use the shared acquisition with the fibre directions
 // mapped by M^T, and the isotropic signal (and the model-3 R term) the
 // voxel's own b values, kept per row in LDS.
-template <int K, int VPL, int MODEL, bool RIC, bool GN = false>
+template <int K, int VPL, int MODEL, bool RIC, bool GN = false, bool FULL = false>
 struct Chain {
   // lane-resident volume state, volume i = rl + 16 t.  One per-volume
   // array lives in the wave's LDS block `vol` instead of registers (18
@@ -199,8 +202,14 @@ struct Chain {
   // the isotropic signal of the Gaussian chain, the data of the Rician one.
   // The --gradnonlin kernels keep both in registers (their LDS holds the
   // rows' b values).
-  static constexpr bool ISO_LDS = !GN && !RIC, Y_LDS = !GN && RIC;
-  float r[Y_LDS ? 1 : VPL];  // Gaussian: y - S0*M; Rician: y
+  // Tiles of up to 5 volumes per lane keep everything in registers, the
+  // acquisition and the stick arguments too: their proposals are short chains
+  // of dependent operations, where each LDS read adds its latency (2,000
+  // voxels of 69 volumes, model 1: 5.5 -> 4.4 ms).  At 10 volumes per lane and
+  // K=3 the registers run out (48 spilled).
+  static constexpr bool SMALL = VPL <= 5;
+  static constexpr bool ISO_LDS = !GN && !RIC && !SMALL, Y_LDS = !GN && RIC && !SMALL;
+  float r[Y_LDS ? 1 : VPL];  // Gaussian: y - S0*M; Rician: -2 y
   float M[VPL];
   float iso_r[ISO_LDS ? 1 : VPL];
   float s[K][VPL];
@@ -213,6 +222,8 @@ struct Chain {
   static constexpr int HELD = VPL * (2 * K + 3 + !ISO_LDS + RIC);  // floats a lane holds in a diffusivity proposal
   static constexpr bool U_LDS = HELD <= (RIC ? 130 : 162) * (VPL > 18 ? 2 : 1);
   float* sk;
+  float ur[SMALL ? K : 1][SMALL ? VPL : 1];
+  float4 ga[SMALL ? VPL : 1];
   float ell[RIC ? VPL : 1];
   // isotropic signal per b-shell (acquisitions with <= 16 distinct b values):
   // sh[i] is the shell of volume i, shb[l] its b value, isot the row's table
@@ -238,7 +249,7 @@ struct Chain {
   int nv;       // slots of this lane that hold a real volume (rl + 16 t < N)
   int rl;
   // slot 0 holds b = 0 volumes only (see stage_acq): the moves that leave
-  // their signals at 1 skip it (18-volume tiles only)
+  // their signals at 1 skip it (ZERO_SLOT tiles only)
   bool z0;
   FDT_DEV bool skip(int t) const { return ZERO_SLOT<VPL> && t == 0 && z0; }
   // options
@@ -272,6 +283,17 @@ struct Chain {
   template <int SL> FDT_DEV void accept() { accm |= 1u << SL; }
 
   FDT_DEV float& ldsk(int k, int t) const { return sk[(k * VPL + t) * 64]; }
+  // stick-signal argument of fibre k at slot t
+  FDT_DEV float& arg(int k, int t) {
+    if constexpr (SMALL) return ur[k][t];
+    else return ldsk(k, t);
+  }
+  // acquisition of slot t
+  FDT_DEV float4 grad(int t) const {
+    if constexpr (SMALL) return ga[t];
+    else return acq[rl + 16 * t];
+  }
+  FDT_DEV static void fence() { if constexpr (!SMALL) reload_acq(); }
   FDT_DEV float& isov(int t) {
     if constexpr (ISO_LDS) return vol[t * 64];
     else return iso_r[t];
@@ -280,11 +302,14 @@ struct Chain {
     if constexpr (ISO_LDS) return vol[t * 64];
     else return iso_r[t];
   }
-  // the Rician chain's data of slot t
-  FDT_DEV float yv(int t) const {
+  // the Rician chain's data of slot t, held as -2 y (exact): with h = -tau p / 2
+  // the argument of log I0 is h (-2 y) and the quadratic part h p
+  FDT_DEV float ym2(int t) const {
     if constexpr (Y_LDS) return vol[t * 64];
     else return r[t];
   }
+  FDT_DEV float yv(int t) const { return -0.5f * ym2(t); }
+  float yy;  // Rician: sum of y^2 over the row's volumes
   // unit directions of the row's fibres (from the theta / phi slots)
   struct Dirs {
     float x[K][3];
@@ -308,7 +333,8 @@ struct Chain {
   // so the f0, f and angle proposals, whose per-volume change is then exactly
   // 0 there, need no mask; the S0 and diffusivity proposals, where the
   // mixture at a padding slot moves by rounding, and every Rician term do.
-  FDT_DEV float mask(int t, float x) const { return t < nv ? x : 0.0f; }
+  // FULL: the tile has no padding (N = 16 VPL).
+  FDT_DEV float mask(int t, float x) const { return FULL || t < nv ? x : 0.0f; }
   // sum of the fractions (f0 first, the order of the reference's sums)
   FDT_DEV float sum_fractions() const {
     float q = f0;
@@ -438,16 +464,11 @@ struct Chain {
     if constexpr (RIC) {
       const float tn = cand<SL_TAU>();
       if (tn <= 0.0f) return;
-      float a = 0.0f, yy = 0.0f, en[VPL];
-#pragma unroll
-      for (int t = 0; t < VPL; ++t) {
-        const float y = yv(t);
-        yy += mask(t, y * y);
-      }
+      float a = 0.0f, en[VPL];
       ric_terms<true>([&](int t) { return S0 * M[t]; }, tn, en, a);
       a = row_sum16(a);  // change of the stored terms (the running sum's)
       // the -tau y^2 / 2 part of the full terms moves with tau too
-      float dE = -Nf * (flog(tn) - flog(tau)) - fmaf(-0.5f * (tn - tau), row_sum16(yy), a);
+      float dE = -Nf * (flog(tn) - flog(tau)) - fmaf(-0.5f * (tn - tau), yy, a);
       if (dE < -lu) {
 #pragma unroll
         for (int t = 0; t < VPL; ++t) ell[t] = en[t];
@@ -491,7 +512,7 @@ struct Chain {
   // variant only; no per-slot branch)
   template <bool NI, class F>
   FDT_DEV void by_shells(F&& f) const {
-    if constexpr (NI && !GN) {
+    if constexpr (NI && !GN && !(SMALL && MODEL == 1)) {
       if (nshell) f(std::true_type{});
       else f(std::false_type{});
     } else f(std::false_type{});
@@ -505,19 +526,21 @@ struct Chain {
   // ALL: also slot 0 of b = 0 volumes (the S0 and tau moves).
   template <bool ALL, class P>
   FDT_DEV void ric_terms(P&& p, float tv, float (&en)[RIC ? VPL : 1], float& a) const {
+    const float th = -0.5f * tv;
 #pragma unroll
     for (int t0 = 0; t0 < VPL; t0 += RG) {
-      float q[RG], x[RG];
+      float q[RG], h[RG], x[RG];
       bool sm = false;
       auto out = [&](int t) { return t >= VPL || (!ALL && skip(t)); };
 #pragma unroll
       for (int i = 0; i < RG; ++i) {
         const int t = t0 + i;
-        q[i] = x[i] = 0.0f;
+        q[i] = h[i] = x[i] = 0.0f;
         if (out(t)) continue;
         q[i] = p(t);
-        x[i] = tv * q[i] * yv(t);
-        sm = sm || (t < nv && fabsf(x[i]) < 3.75f);
+        h[i] = th * q[i];
+        x[i] = h[i] * ym2(t);
+        sm = sm || ((FULL || t < nv) && fabsf(x[i]) < 3.75f);
       }
       if (__builtin_amdgcn_ballot_w64(sm)) {
 #pragma unroll
@@ -532,7 +555,7 @@ struct Chain {
       for (int i = 0; i < RG; ++i) {
         const int t = t0 + i;
         if (out(t)) continue;
-        en[t] = fmaf(-0.5f * (tv * q[i]), q[i], x[i]);
+        en[t] = fmaf(h[i], q[i], x[i]);
         a += mask(t, en[t] - ell[t]);
       }
     }
@@ -557,7 +580,7 @@ struct Chain {
       if (rl == SL_R) { sprn = prn; sdp = prn - sprior; }
     }
     const SigC cn = aniso_coef<MODEL>(dn, dsn, Rn), ci = iso_coef<MODEL>(dn, dsn);
-    reload_acq();
+    fence();
     constexpr bool KEEP_M = U_LDS || RIC;
     float a = 0.0f, mn[KEEP_M ? VPL : 1], en[RIC ? VPL : 1], sn[U_LDS ? K : 1][VPL];
     Dirs D;
@@ -578,10 +601,10 @@ struct Chain {
         if (t >= VPL) return;
         if constexpr (NA && U_LDS) {
 #pragma unroll
-          for (int k = 0; k < K; ++k) u[k][t] = ldsk(k, t);
+          for (int k = 0; k < K; ++k) u[k][t] = arg(k, t);
         }
-        if constexpr (NA && !U_LDS) g[t] = acq[rl + 16 * t];
-        if constexpr ((NA && SA == 2) || (NI && !SH)) b[t] = bv(t, acq[rl + 16 * t]);
+        if constexpr (NA && !U_LDS) g[t] = grad(t);
+        if constexpr ((NA && SA == 2) || (NI && !SH)) b[t] = bv(t, grad(t));
         if constexpr (SH) iso[t] = isot[si[t]];
         else if constexpr (!NI) iso[t] = isov(t);
       };
@@ -609,13 +632,13 @@ struct Chain {
         if constexpr (!RIC) qd.add(r[t], mask(t, m - M[t]));
         // the gamma form has several temporaries per volume and signal: keep
         // the scheduler from overlapping many volumes of it (register spills)
-        if constexpr ((NA && SA == 1) || (NI && SI == 1)) reload_acq();
+        if constexpr ((NA && SA == 1) || (NI && SI == 1)) fence();
       }
     });
     if constexpr (RIC) ric_terms<false>([&](int t) { return S0 * mn[t]; }, tau, en, a);
     a = RIC ? row_sum16(a) : qd.delta(S0);
     if (dlik(a) + dprior<SL>() < -lu) {
-      reload_acq();
+      fence();
       by_shells<NI>([&](auto SHc) {
 #pragma unroll
         for (int t = 0; t < VPL; ++t) {
@@ -623,7 +646,7 @@ struct Chain {
           if constexpr (NI) {
             if constexpr (decltype(SHc)::value) isov(t) = isot[sh[rl + 16 * t]];
             else {
-              const float b = bv(t, acq[rl + 16 * t]);
+              const float b = bv(t, grad(t));
               isov(t) = sig<SI>(ci, b, b);
             }
           }
@@ -658,13 +681,13 @@ struct Chain {
     const float sp_ = IS_TH ? sp : sa, cp_ = IS_TH ? cp : cs;
     float x0 = st_ * cp_, x1 = st_ * sp_, x2 = ct_;
     xform(x0, x1, x2);
-    reload_acq();
+    fence();
     float sn[VPL], un[U_LDS ? VPL : 1], qv[VPL], en[RIC ? VPL : 1];
     float a = 0.0f;
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
       if (skip(t)) continue;
-      float4 g = acq[rl + 16 * t];
+      const float4 g = grad(t);
       float dp = fmaf(g.x, x0, fmaf(g.y, x1, g.z * x2));
       const float u = g.w * dp * dp;
       if constexpr (U_LDS) un[t] = u;
@@ -687,7 +710,7 @@ struct Chain {
         M[t] = fmaf(fk[k], qv[t], M[t]);
         if constexpr (RIC) ell[t] = en[t]; else r[t] = fmaf(-c, qv[t], r[t]);
         s[k][t] = sn[t];
-        if constexpr (U_LDS) ldsk(k, t) = un[t];
+        if constexpr (U_LDS) arg(k, t) = un[t];
       }
       like += (double)a;
       if constexpr (IS_TH) { st = sa; ct = cs; } else { sp = sa; cp = cs; }
@@ -762,7 +785,7 @@ struct ChainLds {
 // in order, padding last), so that slot 0 of every row holds b = 0 volumes
 // only, and those proposals skip slot 0.  The likelihood is the same sum over
 // the same volumes; with fewer than 16 the order is the acquisition's.  Only
-// the 18-volume tile does this (ZERO_SLOT).  With --gradnonlin the per-voxel
+// the 14- and 18-volume tiles do this (ZERO_SLOT).  With --gradnonlin the per-voxel
 // b values are b |(I+L) g|^2, zero exactly where the shared table's are, and
 // the rows read them in the staged order.
 constexpr int ZC_CHUNKS = 8;  // 64-volume chunks of the largest table (16 x 32)
@@ -831,9 +854,9 @@ FDT_DEV bool zero_slot0(const ChainLds& L) {
 // :507-1474, run twice by CUDA/runmcmc.cu:108-316).  GN (--gradnonlin): the
 // chain reads its voxel's own corrected acquisition from a.acqv (the reference
 // indexes per-voxel bvals/alpha/beta with posBV, :266, :711).
-template <int K, int VPL, int MODEL, bool RIC, bool GN = false>
+template <int K, int VPL, int MODEL, bool RIC, bool GN = false, bool FULL = false>
 FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
-  using C = Chain<K, VPL, MODEL, RIC, GN>;
+  using C = Chain<K, VPL, MODEL, RIC, GN, FULL>;
   const int lane = __lane_id();
   const int rl = lane & 15;
   const float4* sacq = L.acq;
@@ -842,6 +865,10 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
   c.acq = sacq;
   c.sk = L.sk + (threadIdx.x >> 6) * (K * VPL * 64) + lane;
   c.vol = L.vol ? L.vol + (threadIdx.x >> 6) * (VPL * 64) + lane : nullptr;
+  if constexpr (C::SMALL) {
+#pragma unroll
+    for (int t = 0; t < VPL; ++t) c.ga[t] = sacq[rl + 16 * t];
+  }
   c.sh = L.sh;
   c.shb = L.shb;
   c.isot = GN ? L.iso : L.iso + (threadIdx.x >> 4) * 16;
@@ -970,24 +997,28 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
     const typename C::Dirs D = c.dirs();
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
-      float4 g = sacq[rl + 16 * t];
+      const float4 g = c.grad(t);
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         float dp = fmaf(g.x, D.x[k][0], fmaf(g.y, D.x[k][1], g.z * D.x[k][2]));
         const float u = g.w * dp * dp;
-        if constexpr (C::U_LDS) c.ldsk(k, t) = u;
+        if constexpr (C::U_LDS) c.arg(k, t) = u;
         c.s[k][t] = sig<STICK_KIND<MODEL>>(c.ca, u, c.bv(t, g));
       }
     }
 #pragma unroll
-    for (int t = 0; t < VPL; ++t) { float b = c.bv(t, sacq[rl + 16 * t]); c.isov(t) = sig<ISO_KIND<MODEL>>(ci, b, b); }
+    for (int t = 0; t < VPL; ++t) { float b = c.bv(t, c.grad(t)); c.isov(t) = sig<ISO_KIND<MODEL>>(ci, b, b); }
   }
   if constexpr (RIC) {
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
-      if constexpr (C::Y_LDS) c.vol[t * 64] = y[t];
-      else c.r[t] = y[t];
+      if constexpr (C::Y_LDS) c.vol[t * 64] = -2.0f * y[t];
+      else c.r[t] = -2.0f * y[t];
     }
+    float yy = 0.0f;
+#pragma unroll
+    for (int t = 0; t < VPL; ++t) yy += c.mask(t, square(y[t]));
+    c.yy = row_sum16(yy);
   }
   c.rebuild(y);
 
@@ -1081,7 +1112,7 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
         const float e = c.yv(t) - S0 * c.M[t];
-        acc += c.mask(t, e * e);
+        acc += c.mask(t, square(e));
       }
       ss = (double)row_sum16(acc);
     } else {

@@ -15,16 +15,17 @@ __device__ inline int xcd_tile(int b, int nb) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + l;
 }
 
-template <int K, int VPL, int MODEL, bool RIC, bool GN>
+template <int K, int VPL, int MODEL, bool RIC, bool GN, bool FULL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VPL <= 18 ? 2 : 1, 2))) void mcmc_kernel(McmcArgs a) {
   __shared__ float4 sacq[16 * VPL];
-  __shared__ float sba[4 * K * VPL * 64];
+  constexpr bool SMALL = Chain<K, VPL, MODEL, RIC, GN, FULL>::SMALL;  // state in registers
+  __shared__ float sba[SMALL ? 1 : 4 * K * VPL * 64];
   __shared__ int ssh[GN ? 1 : 16 * VPL];
   __shared__ float sshb[16];
   __shared__ float siso[GN ? 1 : 16 * 16];
   __shared__ float sbp[GN ? 16 * 16 * VPL : 1];
   __shared__ float sgd[GN ? 16 * 9 : 1];
-  __shared__ float svol[GN ? 1 : 4 * VPL * 64];
+  __shared__ float svol[GN || SMALL ? 1 : 4 * VPL * 64];
   constexpr bool ZS = ZERO_SLOT<VPL>;
   __shared__ int sperm[ZS ? 16 * VPL : 1];
   __shared__ int szc[ZS ? ZC_CHUNKS : 1];
@@ -33,7 +34,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VPL <= 18 ?
   stage_acq<VPL>(a, L);
   __syncthreads();
   const int i = xcd_tile(blockIdx.x, gridDim.x) * 16 + (threadIdx.x >> 4);
-  if (i < a.nvox) run_chain<K, VPL, MODEL, RIC, GN>(a, a.list ? a.list[i] : i, L);
+  if (i < a.nvox) run_chain<K, VPL, MODEL, RIC, GN, FULL>(a, a.list ? a.list[i] : i, L);
 }
 
 }  // namespace fdt
@@ -57,8 +58,14 @@ namespace {
 template <int K, int MODEL, bool RIC>
 hipError_t launch_model(const fdt::McmcArgs* a, hipStream_t s) {
   dim3 grid((a->nvox + 15) / 16), block(256);
-  if (a->acqv) hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, true>), grid, block, 0, s, *a);
-  else hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false>), grid, block, 0, s, *a);
+  // 288 volumes (18 b = 0 and 270 directions) fill the 18-volume tile: a kernel without the padding masks there
+  // (250,968 voxels, model 2: 1,013 -> 1,001 ms; model-3 Rician chains of 16,384 voxels, with the halved products
+  // of their terms: 202 -> 185 ms)
+  constexpr bool CAN_FULL = FDT_VPL == 18;
+  if (a->acqv) hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, true, false>), grid, block, 0, s, *a);
+  else if (CAN_FULL && a->N == 16 * FDT_VPL)
+    hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false, CAN_FULL>), grid, block, 0, s, *a);
+  else hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false, false>), grid, block, 0, s, *a);
   return hipGetLastError();
 }
 template <int K, bool RIC>
