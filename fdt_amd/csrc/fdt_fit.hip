@@ -52,9 +52,13 @@ FDT_DEV T rsum(T v) {
 //   PVM_single   CUDA/PVM_single.cu:107-373
 //   PVM_single_c CUDA/PVM_single_c.cu:104-514
 //   PVM_multi    CUDA/PVM_multi.cu:19-466
+// KIND carries the PVM_multi variant G (0 gamma, 1 gamma for the ball only, 2
+// zeppelin) as KIND_MULTI + G.
 template <class T, int KIND, int K, bool F0>
 struct Mdl {
-  static constexpr int FB = (KIND == KIND_MULTI) ? 3 : 2;
+  static constexpr bool MULTI = KIND >= KIND_MULTI;
+  static constexpr int G = KIND - KIND_MULTI;
+  static constexpr int FB = MULTI ? 3 : 2;
   static constexpr int NP = FB + 3 * K + (F0 ? 1 : 0);
   T fs[K], x0[K], x1[K], x2[K], sth[K], cth[K], sph[K], cph[K];
   T fder[K][K];
@@ -62,7 +66,6 @@ struct Mdl {
   // per-stage constants of the Jacobian rows, hoisted out of the volume loop:
   // d f / d x of the f = x2f(x) fractions (and of f0), and 1 / p[0]
   T dfx[K], dfx0, ip0;
-  int G;
   T Rv, invR;
   // exp / log of the model and Jacobian rows: the hardware exp2 / log2 with one
   // scaling in FP32 (a few ulp, below the FP32 noise of the fit); exp_d /
@@ -159,18 +162,22 @@ struct Mdl {
   }
 
   FDT_DEV T aniso(T b, T dp) const {
-    if constexpr (KIND != KIND_MULTI) return ex(-b * d * dp * dp);
+    if constexpr (!MULTI) return ex(-b * d * dp * dp);
     else {
-      if (G == 1) return ex(-b * a * bb * dp * dp);
-      if (G == 2) return ex(-b * T(3) * a * bb * invR * ((T(1) - Rv) * dp * dp + Rv));
-      return ex(-a * lg(T(1) + b * bb * (dp * dp)));
+      if constexpr (G == 1) return ex(-b * a * bb * dp * dp);
+      else if constexpr (G == 2) return ex(-b * T(3) * a * bb * invR * ((T(1) - Rv) * dp * dp + Rv));
+      else return ex(-a * lg(T(1) + b * bb * (dp * dp)));
     }
   }
 
+  static FDT_DEV T product(T x, T y) {
+#pragma clang fp contract(off)
+    return x * y;
+  }
   // isotropic signal at b (a function of b alone: evaluated once per b shell
   // where the acquisition has shells)
   FDT_DEV T iso_val(T b) const {
-    if constexpr (KIND == KIND_MULTI) return ex(-a * lg(T(1) + b * bb));
+    if constexpr (MULTI) return ex(-a * lg(T(1) + b * bb));
     else return ex(-b * d);
   }
   FDT_DEV T pred_iso(const T* p, T b, T gx, T gy, T gz, T iso) const {
@@ -180,7 +187,7 @@ struct Mdl {
       T dp = gx * x0[k] + gy * x1[k] + gz * x2[k];
       err += fs[k] * aniso(b, dp);
     }
-    if constexpr (KIND == KIND_MULTI) {
+    if constexpr (MULTI) {
       T S0 = fabs(p[0]);
       if constexpr (F0) return S0 * (tf0 + ((T(1) - sumf - tf0) * iso + err));
       else return S0 * ((T(1) - sumf) * iso + err);
@@ -189,7 +196,11 @@ struct Mdl {
       else return p[0] * ((T(1) - sumf) * iso + err);
     }
   }
-  FDT_DEV T pred(const T* p, T b, T gx, T gy, T gz) const { return pred_iso(p, b, gx, gy, gz, iso_val(b)); }
+  FDT_DEV T pred(const T* p, T b, T gx, T gy, T gz) const {
+    if constexpr (G == 2 || (G == 0 && std::is_same<T, float>::value)) {  // here b bb has its own rounding (the stick exponents share it)
+      return pred_iso(p, b, gx, gy, gz, ex(-a * lg(T(1) + product(b, bb))));
+    } else return pred_iso(p, b, gx, gy, gz, iso_val(b));
+  }
 
   // Jacobian row for the gradient (Jg); the Hessian row equals it except in
   // column 0 for PVM_multi (CUDA/PVM_multi.cu:317 vs :451), returned in J0h.
@@ -273,13 +284,13 @@ struct Mdl {
         T dp1t = cth[k] * (gx * cph[k] + gy * sph[k]) - gz * sth[k];
         T dp1p = sth[k] * (-gx * sph[k] + gy * cph[k]);
         T an, an_a, an_b, an_th, an_ph;
-        if (G == 1) {
+        if constexpr (G == 1) {
           an = ex(-b * a * bb * dp * dp);
           an_a = -b * bb * dp * dp * an;
           an_b = -b * a * dp * dp * an;
           an_th = T(-2) * b * a * bb * dp * dp1t * an;
           an_ph = T(-2) * b * a * bb * dp * dp1p * an;
-        } else if (G == 2) {
+        } else if constexpr (G == 2) {
           T t = (T(1) - Rv) * dp * dp + Rv;
           an = ex(-b * T(3) * a * bb * invR * t);
           T qa = b * T(3) * bb * invR * t;
@@ -1039,11 +1050,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_sam
     R.isot = sisot + (threadIdx.x >> 4) * 16;
   }
   M m0;
-  m0.G = a.G;
   m0.Rv = (T)a.R;
   m0.invR = T(1) / (T(2) * (T)a.R + T(1));
   Mdl<TC, KIND, K, F0> mc0;
-  mc0.G = a.G;
   mc0.Rv = (TC)a.R;
   mc0.invR = TC(1) / (TC(2) * (TC)a.R + TC(1));
   const int count = a.count ? *a.count : a.nvox;
@@ -1076,7 +1085,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_sam
       if (a.init == INIT_BUF) {
 #pragma unroll
         for (int i = 0; i < NP; ++i) S.p[i] = (TC)a.in[(size_t)vox * a.in_np + i];
-      } else if constexpr (KIND == KIND_MULTI) {
+      } else if constexpr (KIND >= KIND_MULTI) {
         TC s1[NP - 1];
 #pragma unroll
         for (int i = 0; i < NP - 1; ++i) s1[i] = (TC)a.in[(size_t)vox * a.in_np + i];
@@ -1295,6 +1304,10 @@ hipError_t launch_kind(const fdt::LmArgs* a, int kind, int f0, hipStream_t s) {
   using namespace fdt;
   if (kind == KIND_SINGLE) return f0 ? launch_lm<KIND_SINGLE, true, GN>(a, s) : launch_lm<KIND_SINGLE, false, GN>(a, s);
   if (kind == KIND_SINGLE_C) return f0 ? launch_lm<KIND_SINGLE_C, true, GN>(a, s) : launch_lm<KIND_SINGLE_C, false, GN>(a, s);
+  if (kind == KIND_MULTI && a->G == 1)
+    return f0 ? launch_lm<KIND_MULTI + 1, true, GN>(a, s) : launch_lm<KIND_MULTI + 1, false, GN>(a, s);
+  if (kind == KIND_MULTI && a->G == 2)
+    return f0 ? launch_lm<KIND_MULTI + 2, true, GN>(a, s) : launch_lm<KIND_MULTI + 2, false, GN>(a, s);
   if (kind == KIND_MULTI) return f0 ? launch_lm<KIND_MULTI, true, GN>(a, s) : launch_lm<KIND_MULTI, false, GN>(a, s);
   return hipErrorInvalidValue;
 }
