@@ -3,7 +3,8 @@
 // One voxel per 16-lane DPP row, four voxels per wave64, 16 per 256-thread
 // workgroup.  Launches are persistent: each row takes a voxel from a device
 // work queue, runs one LM stage on it to convergence and takes the next, so a
-// slow voxel never holds back the rest of its wave.  The stages of the
+// slow voxel never holds back the rest of its wave; launches of few voxels give
+// each a wave (lm_wave_kernel).  The stages of the
 // reference's fit() (CUDA/xfibres_gpu.cu:173-348) are separate launches:
 //   tensor fit (DTI::linfit, diffmodels.cc:17-46, done per voxel on the host
 //   by the reference, CUDA/diffmodels.cu:57-94) -> start values
@@ -21,6 +22,7 @@
 // mode).
 #include "fdt_device.h"
 #include "fdt_kernels.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace fdt {
@@ -38,7 +40,23 @@ struct Row {
   const int* sh = nullptr;
   const float* shb = nullptr;
   double* isot = nullptr;
+  // the wave's LDS block for the cooperative mode (row_cost_w, row_normal_eq_w)
+  char* wave = nullptr;
 };
+
+// LDS operations of one wave execute in order: only the compiler has to be
+// kept from moving them across
+FDT_DEV void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// a product rounded on its own, not contracted into a sum
+template <class T>
+FDT_DEV T product(T x, T y) {
+#pragma clang fp contract(off)
+  return x * y;
+}
 
 template <class T>
 FDT_DEV T rsum(T v) {
@@ -170,10 +188,6 @@ struct Mdl {
     }
   }
 
-  static FDT_DEV T product(T x, T y) {
-#pragma clang fp contract(off)
-    return x * y;
-  }
   // isotropic signal at b (a function of b alone: evaluated once per b shell
   // where the acquisition has shells)
   FDT_DEV T iso_val(T b) const {
@@ -360,6 +374,41 @@ FDT_DEV double row_cost(const Row& R, const M& m, const T* p) {
   return row_sum16_d(c);
 }
 
+// The cooperative kernel (lm_wave_kernel) gives a voxel all 64 lanes of a wave:
+// where there are few voxels, what bounds the fit is the latency of one loop
+// trip, most of it the model at N / 16 volumes per lane.  The rows evaluate the
+// model rows of different volumes and hand them over in LDS; every sum over
+// volumes is then taken in the order of the one-row kernel, so the fit is the
+// same to the last bit.
+//
+// row_cost with the volumes of lane l dealt out over the four rows
+template <class T, class M>
+FDT_DEV double row_cost_w(const Row& R, const M& m, const T* p) {
+  T* eb = reinterpret_cast<T*>(R.wave);
+  const int row = __lane_id() >> 4;
+  if (R.nshell) {
+    if (R.rl < R.nshell) R.isot[R.rl] = (double)m.iso_val((T)R.shb[R.rl]);
+    wave_order();
+    for (int i = R.rl + 16 * row; i < R.N; i += 64) {
+      float4 q = R.acq[i];
+      eb[i] = m.pred_iso(p, (T)q.w, (T)q.x, (T)q.y, (T)q.z, (T)R.isot[R.sh[i]]) - (T)R.y[i];
+    }
+  } else {
+    for (int i = R.rl + 16 * row; i < R.N; i += 64) {
+      float4 q = R.acq[i];
+      eb[i] = m.pred(p, (T)q.w, (T)q.x, (T)q.y, (T)q.z) - (T)R.y[i];
+    }
+  }
+  wave_order();
+  double c = 0.0;
+  for (int i = R.rl; i < R.N; i += 16) {
+    const T e = eb[i];
+    c += (double)e * (double)e;
+  }
+  wave_order();
+  return row_sum16_d(c);
+}
+
 // LU with partial pivoting and substitution, row i of the matrix and entry i
 // of the right-hand side in lane i of the row.  The elimination order, the
 // pivot rule (first maximum of the column at and below the diagonal; after a
@@ -476,6 +525,91 @@ FDT_DEV void row_normal_eq(const Row& R, const Mdl<T, KIND, K, F0>& m, const T* 
   for (int c = 0; c < NP; ++c) Hrow[c] = (double)hsel[c];
 }
 
+// Row stride of the wave's LDS block in row_normal_eq_w: whole 16-byte units, an odd
+// number of 4-bank groups apart, so that the 16 lanes' vector reads meet no bank twice
+template <class T> constexpr int WSTRIDE = std::is_same<T, float>::value ? 20 : 18;
+template <class T, class TC> constexpr size_t wave_bytes(int N) {
+  const size_t a = 64 * WSTRIDE<T> * sizeof(T), b = (size_t)N * sizeof(TC);
+  return ((a > b ? a : b) + 15) / 16 * 16;
+}
+
+// row_normal_eq in the cooperative mode: in steps of four volumes per lane,
+// each row evaluates the Jacobian rows of one of them and then adds all four
+// to its own rows a = row, row + 4, ... of J^T J and J^T r (whole rows: the
+// entries below the diagonal are the products above it the other way round).
+template <class T, int KIND, int K, bool F0>
+FDT_DEV void row_normal_eq_w(const Row& R, const Mdl<T, KIND, K, F0>& m, const T* p,
+                             double (&Hrow)[Mdl<T, KIND, K, F0>::NP], double& grow) {
+  constexpr int NP = Mdl<T, KIND, K, F0>::NP, NA = (NP + 3) / 4, ST = WSTRIDE<T>;
+  static_assert(NP + 2 <= 16, "Jacobian row longer than its LDS slot");
+  T* jb = reinterpret_cast<T*>(R.wave);
+  const int row = __lane_id() >> 4;
+  T g[NA], h[NA][NP];
+#pragma unroll
+  for (int q = 0; q < NA; ++q) {
+    g[q] = T(0);
+#pragma unroll
+    for (int c = 0; c < NP; ++c) h[q][c] = T(0);
+  }
+  for (int i0 = R.rl; i0 - R.rl < R.N; i0 += 64) {
+    const int i = i0 + 16 * row;
+    if (i < R.N) {
+      float4 q = R.acq[i];
+      T Jg[NP], J0h;
+      T sig = m.jrow(p, (T)q.w, (T)q.x, (T)q.y, (T)q.z, Jg, J0h);
+      // slot: the Hessian's Jacobian row, then the gradient's entry 0 and the residual
+      T v[16];
+#pragma unroll
+      for (int c = 0; c < NP; ++c) v[c] = c == 0 ? J0h : Jg[c];
+      v[NP] = Jg[0];
+      v[NP + 1] = sig - (T)R.y[i];
+      T* d = jb + (16 * row + R.rl) * ST;
+#pragma unroll
+      for (int c = 0; c < NP + 2; ++c) d[c] = v[c];
+    }
+    wave_order();
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if (i0 + 16 * w >= R.N) continue;
+      const T* d = jb + (16 * w + R.rl) * ST;
+      T v[NP];
+#pragma unroll
+      for (int c = 0; c < NP; ++c) v[c] = d[c];
+      const T diff = d[NP + 1];
+#pragma unroll
+      for (int q = 0; q < NA; ++q) {
+        const int a = row + 4 * q;
+        const T ja = d[a < NP ? a : 0], jg = d[a == 0 ? NP : (a < NP ? a : 0)];
+        g[q] += jg * diff;
+#pragma unroll
+        for (int c = 0; c < NP; ++c) h[q][c] += ja * v[c];
+      }
+    }
+    wave_order();
+  }
+  // row a of the sums to lane a of every row
+#pragma unroll
+  for (int q = 0; q < NA; ++q) {
+    const int a = row + 4 * q;
+    const T ga = T(2) * rsum<T>(g[q]);
+    T hv[NP];
+#pragma unroll
+    for (int c = 0; c < NP; ++c) hv[c] = T(2) * rsum<T>(h[q][c]);
+    if (R.rl == 0) {
+      T* d = jb + a * ST;
+#pragma unroll
+      for (int c = 0; c < NP; ++c) d[c] = hv[c];
+      d[NP] = ga;
+    }
+  }
+  wave_order();
+  const T* d = jb + R.rl * ST;
+#pragma unroll
+  for (int c = 0; c < NP; ++c) Hrow[c] = (double)d[c];
+  grow = (double)d[NP];
+  wave_order();
+}
+
 // The Levenberg loop of CUDA/levenberg_marquardt.cu:24-115 as a resumable
 // per-row state: lambda0 = 0.1, /10 after a success, x10 after a failure (the
 // Hessian diagonal carries lambda - lambda_old), relative cost test 1e-8,
@@ -497,15 +631,19 @@ struct LmState {
   int niter, total;
   bool success;
 
+  template <bool W>
   FDT_DEV void begin(const Row& R, const Mdl<TC, KIND, K, F0>& mc0) {
     Mdl<TC, KIND, K, F0> m = mc0;
     m.prep(p);
-    pcf = row_cost<TC>(R, m, p);
+    if constexpr (W) pcf = row_cost_w<TC>(R, m, p);
+    else pcf = row_cost<TC>(R, m, p);
     lambda = 0.1; olambda = 0.0;
     niter = 0; total = 0;
     success = true;
   }
-  // one trip of the loop; returns true when the stage has ended
+  // one trip of the loop; returns true when the stage has ended.  W: all four
+  // rows of the wave hold this voxel.
+  template <bool W>
   FDT_DEV bool step(const Row& R, const Mdl<T, KIND, K, F0>& m0, const Mdl<TC, KIND, K, F0>& mc0) {
     if (success && niter++ >= 200) return true;
     ++total;
@@ -515,7 +653,8 @@ struct LmState {
 #pragma unroll
       for (int i = 0; i < NP; ++i) pj[i] = (T)p[i];
       m.prep(pj);
-      row_normal_eq<T, KIND, K, F0>(R, m, pj, Hrow, grow);
+      if constexpr (W) row_normal_eq_w<T, KIND, K, F0>(R, m, pj, Hrow, grow);
+      else row_normal_eq<T, KIND, K, F0>(R, m, pj, Hrow, grow);
     }
 #pragma unroll
     for (int i = 0; i < NP; ++i) if (R.rl == i) Hrow[i] += (lambda - olambda);
@@ -526,7 +665,9 @@ struct LmState {
     for (int i = 0; i < NP; ++i) st[i] = p[i] - (TC)sol[i];
     Mdl<TC, KIND, K, F0> mc = mc0;
     mc.prep(st);
-    double ncf = row_cost<TC>(R, mc, st);
+    double ncf;
+    if constexpr (W) ncf = row_cost_w<TC>(R, mc, st);
+    else ncf = row_cost<TC>(R, mc, st);
     bool end = false;
     if ((success = (ncf < pcf))) {
       olambda = 0.0;
@@ -579,14 +720,28 @@ FDT_DEV void finalise(T* p) {
     }
   } else if constexpr (KIND == KIND_SINGLE_C) {
     p[1] = p[1] * p[1];
+    T rest = T(1);  // 1 - the fractions before
+    if constexpr (F0 && K > 1) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      T pt = T(1);
+      for (int k = 0; k < K; ++k) {
+        T pt = T(1);
 #pragma unroll
-      for (int j = 0; j < k; ++j) pt -= p[2 + 3 * j];
-      p[2 + 3 * k] = beta2f<T>(p[2 + 3 * k]) * pt;
+        for (int j = 0; j < k; ++j) pt -= p[2 + 3 * j];
+        p[2 + 3 * k] = beta2f<T>(p[2 + 3 * k]) * pt;
+      }
+    } else {
+      // the same recursion with its roundings written out: 1 - s^2 in one, f2 and 1 - f1 - f2 in their own
+      T& pt = rest;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const T sb = sin(p[2 + 3 * k]);
+        const T f = k ? product(product(sb, sb), pt) : sb * sb;
+        pt = k ? pt - f : fma(-sb, sb, T(1));
+        p[2 + 3 * k] = f;
+      }
     }
-    if constexpr (F0) {
+    if constexpr (F0 && K == 1) p[NP - 1] = beta2f<T>(p[NP - 1]) * rest;
+    else if constexpr (F0) {
       T pt = T(1);
 #pragma unroll
       for (int j = 0; j < K; ++j) pt -= p[2 + 3 * j];
@@ -1022,11 +1177,59 @@ FDT_DEV void store_vec(float* dst, const T (&v)[NP], int rl) {
     if (rl == j) dst[j] = (float)v[j];
 }
 
+// The signal row of voxel `vox` to LDS, non-positive samples replaced by the
+// smallest positive one for --rician (remove_NonPositive_entries,
+// CUDA/xfibres_gpu.cu:350-367)
+FDT_DEV void load_signal(const LmArgs& a, int vox, float* ym, int rl) {
+  const float* src = a.data + (size_t)vox * a.N;
+  float mn = 3.0e38f, mx = -3.0e38f, mnp = 3.0e38f;
+  for (int i = rl; i < a.N; i += 16) {
+    float v = src[i];
+    ym[i] = v;
+    mn = fminf(mn, v); mx = fmaxf(mx, v);
+    if (v > 0.0f) mnp = fminf(mnp, v);
+  }
+  if (a.rician) {
+    mn = row_min16(mn); mx = row_max16(mx); mnp = row_min16(mnp);
+    if (mn <= 0.0f && mx > 0.0f)
+      for (int i = rl; i < a.N; i += 16) if (ym[i] <= 0.0f) ym[i] = mnp;
+  }
+}
+// the start vector of voxel `vox`
+template <class TC, int KIND, int K, bool F0, bool GN, int NP>
+FDT_DEV void start_vector(const LmArgs& a, int vox, const Row& R, TC (&p)[NP]) {
+  if (a.init == INIT_BUF) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) p[i] = (TC)a.in[(size_t)vox * a.in_np + i];
+  } else if constexpr (KIND >= KIND_MULTI) {
+    TC s1[NP - 1];
+#pragma unroll
+    for (int i = 0; i < NP - 1; ++i) s1[i] = (TC)a.in[(size_t)vox * a.in_np + i];
+    start_multi<TC, K, F0>(s1, p);
+  } else {
+    Dti dti;
+    if constexpr (GN) dti = dti_row_gn(R);
+    else dti = dti_row(R, a.pinvA);
+    if constexpr (KIND == KIND_SINGLE) start_single<TC, K, F0>(dti, p);
+    else start_single_c<TC, K, F0>(dti, R, p);
+  }
+}
+// the finalised vector and iteration count of a finished stage
+template <class TC, int KIND, int K, bool F0, int NP>
+FDT_DEV void store_result(const LmArgs& a, int vox, TC (&p)[NP], int total, int rl) {
+  finalise<TC, KIND, K, F0>(p);
+  store_vec<NP>(a.out + (size_t)vox * a.out_np, p, rl);
+  if (a.set_f0_slot && rl == 15) a.out[(size_t)vox * a.out_np + a.out_np - 1] = 0.001f;
+  if (a.iters && rl == 0) a.iters[vox] = (a.iters_add ? a.iters[vox] : 0) + total;
+}
+
 // GN: --gradnonlin, every voxel reads its own corrected acquisition from
 // a.acqv instead of the workgroup's table in LDS.
 template <class T, class TC, int KIND, int K, bool F0, bool GN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_same<T, TC>::value && std::is_same<T, double>::value ? 1 : 2, 2))) void lm_kernel(LmArgs a) {
   extern __shared__ float4 lds4[];
+  const int count = a.count ? *a.count : a.nvox;
+  if (a.lm && count <= a.wave_max) return;  // lm_wave_kernel's
   float4* sacq = lds4;
   // without shells the table regions are empty (the launcher sizes them)
   const bool shells = !GN && a.nshell > 0;
@@ -1055,10 +1258,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_sam
   Mdl<TC, KIND, K, F0> mc0;
   mc0.Rv = (TC)a.R;
   mc0.invR = TC(1) / (TC(2) * (TC)a.R + TC(1));
-  const int count = a.count ? *a.count : a.nvox;
   LmState<T, TC, KIND, K, F0> S;
   int vox = 0;
   bool fresh = true;
+  // rows of each wave that take voxels: a launch smaller than the grid's rows spreads over its waves
+  const int waves = 4 * gridDim.x;
+  if (((int)__lane_id() >> 4) >= (count + waves - 1) / waves) return;
   for (;;) {
     if (fresh) {
       int q = 0;
@@ -1067,50 +1272,82 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_sam
       if (q >= count) break;
       vox = a.list ? a.list[q] : q;
       if constexpr (GN) R.acq = a.acqv + (size_t)vox * a.acqv_stride;
-      // the voxel's signal row, non-positive samples replaced by the smallest
-      // positive one for --rician (remove_NonPositive_entries, CUDA/xfibres_gpu.cu:350-367)
-      const float* src = a.data + (size_t)vox * a.N;
-      float mn = 3.0e38f, mx = -3.0e38f, mnp = 3.0e38f;
-      for (int i = rl; i < a.N; i += 16) {
-        float v = src[i];
-        ym[i] = v;
-        mn = fminf(mn, v); mx = fmaxf(mx, v);
-        if (v > 0.0f) mnp = fminf(mnp, v);
-      }
-      if (a.rician) {
-        mn = row_min16(mn); mx = row_max16(mx); mnp = row_min16(mnp);
-        if (mn <= 0.0f && mx > 0.0f)
-          for (int i = rl; i < a.N; i += 16) if (ym[i] <= 0.0f) ym[i] = mnp;
-      }
-      if (a.init == INIT_BUF) {
-#pragma unroll
-        for (int i = 0; i < NP; ++i) S.p[i] = (TC)a.in[(size_t)vox * a.in_np + i];
-      } else if constexpr (KIND >= KIND_MULTI) {
-        TC s1[NP - 1];
-#pragma unroll
-        for (int i = 0; i < NP - 1; ++i) s1[i] = (TC)a.in[(size_t)vox * a.in_np + i];
-        start_multi<TC, K, F0>(s1, S.p);
-      } else {
-        Dti dti;
-        if constexpr (GN) dti = dti_row_gn(R);
-        else dti = dti_row(R, a.pinvA);
-        if constexpr (KIND == KIND_SINGLE) start_single<TC, K, F0>(dti, S.p);
-        else start_single_c<TC, K, F0>(dti, R, S.p);
-      }
+      load_signal(a, vox, ym, rl);
+      start_vector<TC, KIND, K, F0, GN>(a, vox, R, S.p);
       if (!a.lm) {
         store_vec<NP>(a.out + (size_t)vox * a.out_np, S.p, rl);
         continue;
       }
-      S.begin(R, mc0);
+      S.template begin<false>(R, mc0);
       fresh = false;
     }
-    if (S.step(R, m0, mc0)) {
-      finalise<TC, KIND, K, F0>(S.p);
-      store_vec<NP>(a.out + (size_t)vox * a.out_np, S.p, rl);
-      if (a.set_f0_slot && rl == 15) a.out[(size_t)vox * a.out_np + a.out_np - 1] = 0.001f;
-      if (a.iters && rl == 0) a.iters[vox] = (a.iters_add ? a.iters[vox] : 0) + S.total;
+    // Rows whose last trip succeeded need new normal equations, the others only
+    // another trial step; a wave pays for the normal equations whenever one row
+    // does.  Successes and failures mostly alternate, so a row that needs them
+    // waits until a second one does (or no other has a trial to make), and the
+    // rows fall into step: per trip of a voxel 2,264 instead of 2,676
+    // instruction slots (a replay of the sequences of 480 multi-shell voxels;
+    // 2,252 for three rows, 2,420 for four).
+    const uint64_t need = __builtin_amdgcn_ballot_w64(S.success), all = __builtin_amdgcn_ballot_w64(true);
+    if (S.success && need != all && __builtin_popcountll(need) < 32) continue;
+    if (S.template step<false>(R, m0, mc0)) {
+      store_result<TC, KIND, K, F0>(a, vox, S.p, S.total, rl);
       fresh = true;
     }
+  }
+}
+
+// A wave per voxel, for launches of at most a.wave_max voxels: two per wave
+// that fits the chip, where a row per voxel would leave most of it idle (the
+// learned start's fallback, small volumes).  A trip at 288 volumes and K=3
+// takes 0.4 of the one-row kernel's time and 1.7 times its lanes' work, so
+// larger launches stay there: 20,011 voxels took 45.1 instead of 40.0 ms when
+// their last ones moved over here.
+template <class T, class TC, int KIND, int K, bool F0, bool GN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_same<T, TC>::value && std::is_same<T, double>::value ? 1 : 2, 2))) void lm_wave_kernel(LmArgs a) {
+  extern __shared__ float4 lds4[];
+  const int count = a.count ? *a.count : a.nvox;
+  if (count > a.wave_max || (int)blockIdx.x * 4 >= count) return;  // lm_kernel's, or more workgroups than voxels
+  const bool shells = !GN && a.nshell > 0;
+  double* sisot = reinterpret_cast<double*>(lds4 + a.N);
+  float* sy = reinterpret_cast<float*>(sisot + (shells ? 4 * 16 : 0));
+  int* ssh = reinterpret_cast<int*>(sy + 4 * ystride(a.N));
+  char* swave = reinterpret_cast<char*>(ssh + (shells ? (a.N + 3) / 4 * 4 : 0));
+  if constexpr (!GN)
+    for (int i = threadIdx.x; i < a.N; i += blockDim.x) {
+      lds4[i] = a.acq[i];
+      if (shells) ssh[i] = a.shell[i];
+    }
+  __syncthreads();
+  using M = Mdl<T, KIND, K, F0>;
+  constexpr int NP = M::NP;
+  const int wave = threadIdx.x >> 6, rl = __lane_id() & 15;
+  float* ym = sy + wave * ystride(a.N);
+  Row R;
+  R.rl = rl; R.N = a.N; R.acq = lds4; R.y = ym;
+  R.wave = swave + wave * wave_bytes<T, TC>(a.N);
+  if (shells) { R.nshell = a.nshell; R.sh = ssh; R.shb = a.shell_b; R.isot = sisot + wave * 16; }
+  M m0;
+  m0.Rv = (T)a.R;
+  m0.invR = T(1) / (T(2) * (T)a.R + T(1));
+  Mdl<TC, KIND, K, F0> mc0;
+  mc0.Rv = (TC)a.R;
+  mc0.invR = TC(1) / (TC(2) * (TC)a.R + TC(1));
+  LmState<T, TC, KIND, K, F0> S;
+  for (;;) {
+    int q = 0;
+    if (__lane_id() == 0) q = atomicAdd(a.queue, 1);
+    q = __builtin_amdgcn_readfirstlane(q);
+    if (q >= count) break;
+    const int vox = a.list ? a.list[q] : q;
+    if constexpr (GN) R.acq = a.acqv + (size_t)vox * a.acqv_stride;
+    load_signal(a, vox, ym, rl);
+    wave_order();
+    start_vector<TC, KIND, K, F0, GN>(a, vox, R, S.p);
+    S.template begin<true>(R, mc0);
+    while (!S.template step<true>(R, m0, mc0)) {}
+    if (__lane_id() < 16) store_result<TC, KIND, K, F0>(a, vox, S.p, S.total, rl);
+    wave_order();
   }
 }
 
@@ -1280,22 +1517,36 @@ using FitReal = std::conditional<FDT_FIT_FP64 == 1, double, float>::type;
 using FitCost = std::conditional<FDT_FIT_FP64 != 0, double, float>::type;
 
 namespace {
-// persistent grid: as many workgroups as stay resident, at most one row per voxel
+// Persistent grids: as many workgroups as stay resident.  Where the number of
+// voxels is on the device (a list), both kernels are launched and one returns.
 template <int KIND, bool F0, bool GN>
 hipError_t launch_lm(const fdt::LmArgs* a, hipStream_t s) {
   auto kern = fdt::lm_kernel<FitReal, FitCost, KIND, FDT_FIT_K, F0, GN>;
+  auto wkern = fdt::lm_wave_kernel<FitReal, FitCost, KIND, FDT_FIT_K, F0, GN>;
   const bool shells = !GN && a->nshell > 0;
-  size_t lds = (size_t)a->N * sizeof(float4) + (size_t)fdt::LM_ROWS * (16 * (((a->N + 15) / 16) | 1)) * sizeof(float) +
-               (shells ? (size_t)fdt::LM_ROWS * 16 * sizeof(double) + (size_t)a->N * sizeof(int) : 0);
-  int dev = 0, cus = 0, per_cu = 0;
+  const size_t N = (size_t)a->N, row = 16 * (((N + 15) / 16) | 1) * sizeof(float), sh = shells ? (N + 3) / 4 * 16 : 0;
+  const size_t lds = N * sizeof(float4) + fdt::LM_ROWS * (row + (shells ? 16 * sizeof(double) : 0)) + sh;
+  const size_t wlds = N * sizeof(float4) + 4 * (row + (shells ? 16 * sizeof(double) : 0)) + sh +
+                      4 * fdt::wave_bytes<FitReal, FitCost>(a->N);
+  int dev = 0, cus = 0, per_cu = 0, wper_cu = 0;
   hipError_t e;
   if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
   if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
   if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, lds)) != hipSuccess) return e;
-  long want = ((long)a->nvox + fdt::LM_ROWS - 1) / fdt::LM_ROWS;
-  long cap = (long)(per_cu > 0 ? per_cu : 1) * cus;
-  int grid = (int)(want < cap ? want : cap);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, s, *a);
+  fdt::LmArgs b = *a;
+  if (a->lm) {
+    if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&wper_cu, wkern, 256, wlds)) != hipSuccess) return e;
+    b.wave_max = 8 * std::max(wper_cu, 1) * cus;
+  }
+  if (!a->lm || a->nvox > b.wave_max) {
+    const long want = ((long)a->nvox + 3) / 4, cap = (long)std::max(per_cu, 1) * cus;
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min(want, cap)), dim3(256), lds, s, b);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if (a->lm && (a->count || a->nvox <= b.wave_max)) {
+    const long want = ((long)a->nvox + 3) / 4, cap = (long)std::max(wper_cu, 1) * cus;
+    hipLaunchKernelGGL(wkern, dim3((unsigned)std::min(want, cap)), dim3(256), wlds, s, b);
+  }
   return hipGetLastError();
 }
 

@@ -41,6 +41,7 @@ struct LmArgs {
   const int* shell;     // [N] b-shell index of each volume, or null
   const float* shell_b; // [16] b value of each shell
   int nshell;           // number of shells (0: none; ignored with acqv)
+  int wave_max;         // launches of at most so many voxels run in lm_wave_kernel alone (set by the launcher)
 };
 
 // implausible-f0 test and refit list (CUDA/xfibres_gpu.cu:216-246, 305-339)
