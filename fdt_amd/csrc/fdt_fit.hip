@@ -1297,12 +1297,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_sam
   }
 }
 
-// A wave per voxel, for launches of at most a.wave_max voxels: two per wave
-// that fits the chip, where a row per voxel would leave most of it idle (the
-// learned start's fallback, small volumes).  A trip at 288 volumes and K=3
-// takes 0.4 of the one-row kernel's time and 1.7 times its lanes' work, so
-// larger launches stay there: 20,011 voxels took 45.1 instead of 40.0 ms when
-// their last ones moved over here.
+// A wave per voxel, for launches of at most a.wave_max voxels (four per wave
+// that fits the chip, two with FP64 normal equations), where a row per voxel
+// leaves most of the chip idle while the longest voxels finish: the learned
+// start's fallback, small volumes, parts.  A trip at 288 volumes and K=3 takes
+// 0.4 of the one-row kernel's time and 1.7 times its lanes' work.  Measured,
+// one-row kernel -> this one, both stages at 288 volumes, K=3: 200 voxels 15.6
+// -> 8.3 ms, 4,000 19.7 -> 14.9, 6,000 25.2 -> 18.7, 8,000 25.8 -> 22.2, 12,000
+// 28.3 either way.  Moving only the last voxels of a larger launch over here
+// did not pay (20,011 voxels: 45.1 instead of 40.0 ms).
 template <class T, class TC, int KIND, int K, bool F0, bool GN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_same<T, TC>::value && std::is_same<T, double>::value ? 1 : 2, 2))) void lm_wave_kernel(LmArgs a) {
   extern __shared__ float4 lds4[];
@@ -1536,7 +1539,8 @@ hipError_t launch_lm(const fdt::LmArgs* a, hipStream_t s) {
   fdt::LmArgs b = *a;
   if (a->lm) {
     if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&wper_cu, wkern, 256, wlds)) != hipSuccess) return e;
-    b.wave_max = 8 * std::max(wper_cu, 1) * cus;
+    // four voxels per resident wave, two where only one wave fits a SIMD (FP64)
+    b.wave_max = (wper_cu > 1 ? 16 * wper_cu : 8) * cus;
   }
   if (!a->lm || a->nvox > b.wave_max) {
     const long want = ((long)a->nvox + 3) / 4, cap = (long)std::max(per_cu, 1) * cus;
