@@ -63,7 +63,7 @@ FDT_VPL_DECL(10)
 FDT_VPL_DECL(14)
 FDT_VPL_DECL(18)
 FDT_VPL_DECL(24)
-FDT_VPL_DECL(27)
+FDT_VPL_DECL(28)
 FDT_VPL_DECL(32)
 }
 
@@ -76,7 +76,7 @@ struct VplEntry { int vpl; mcmc_launch_fn fn; };
 // of 200 volumes in 18 instead of 14
 const VplEntry kVpl[] = {{3, fdt_launch_mcmc_vpl3},   {5, fdt_launch_mcmc_vpl5},   {7, fdt_launch_mcmc_vpl7},
                          {10, fdt_launch_mcmc_vpl10}, {14, fdt_launch_mcmc_vpl14}, {18, fdt_launch_mcmc_vpl18},
-                         {24, fdt_launch_mcmc_vpl24}, {27, fdt_launch_mcmc_vpl27}, {32, fdt_launch_mcmc_vpl32}};
+                         {24, fdt_launch_mcmc_vpl24}, {28, fdt_launch_mcmc_vpl28}, {32, fdt_launch_mcmc_vpl32}};
 
 // the MCMC tile (volumes per lane) for N volumes, at least `force`
 int tile_of(int N, int force) {

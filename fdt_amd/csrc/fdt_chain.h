@@ -194,7 +194,12 @@ FDT_DEV float square(float x) {
 // the stick signals use the shared acquisition with the fibre directions
 // mapped by M^T, and the isotropic signal (and the model-3 R term) the
 // voxel's own b values, kept per row in LDS.
-template <int K, int VPL, int MODEL, bool RIC, bool GN = false, bool FULL = false>
+// ROWS (1 or 2): a voxel's volumes spread over that many consecutive rows of
+// the wave, VPL in each lane; every row holds the slots' state and makes the
+// same decisions.  A sum over volumes runs through the lanes of the first row
+// and on through those of the second, so that it is the one-row sum to the last
+// bit.
+template <int K, int VPL, int MODEL, bool RIC, bool GN = false, bool FULL = false, int ROWS = 1>
 struct Chain {
   // lane-resident volume state, volume i = rl + 16 t.  One per-volume
   // array lives in the wave's LDS block `vol` instead of registers (18
@@ -251,7 +256,82 @@ struct Chain {
   // slot 0 holds b = 0 volumes only (see stage_acq): the moves that leave
   // their signals at 1 skip it (ZERO_SLOT tiles only)
   bool z0;
-  FDT_DEV bool skip(int t) const { return ZERO_SLOT<VPL> && t == 0 && z0; }
+  FDT_DEV bool skip(int t) const { return ROWS == 1 && ZERO_SLOT<VPL> && t == 0 && z0; }
+  // two rows: this lane's slot t is in the slot of b = 0 volumes
+  FDT_DEV bool zero(int t) const { return ROWS > 1 && ZERO_SLOT<VPL * ROWS> && t == 0 && z0; }
+  // A running sum handed from the first row to the second (0 to the first): the
+  // gfx950 row swap exchanges the odd rows of its first operand with the even
+  // rows of its second; clang 20 gives the first result for the second one too,
+  // so only the first is used.
+  static FDT_DEV float next_row(float a) {
+    const auto w = __builtin_amdgcn_permlane16_swap(0, __builtin_bit_cast(int, a), false, false);
+    return __builtin_bit_cast(float, w[0]);
+  }
+  // a total that every lane of the second row holds, to both rows (two voxels per wave)
+  static FDT_DEV float from_last(float a) {
+    const float lo = fdt::rl(a, 16), hi = fdt::rl(a, 48);
+    return __lane_id() < 32 ? lo : hi;
+  }
+  // sum over the voxel's volumes of the row-wise chain f(t, sum so far)
+  // (ALL: slot 0 of b = 0 volumes too)
+  template <bool ALL = false, class F>
+  FDT_DEV float chain_sum(F&& f) const {
+    float a = 0.0f;
+#pragma unroll
+    for (int h = 0; h < ROWS; ++h) {
+      if (h) a = next_row(a);
+#pragma unroll
+      for (int t = 0; t < VPL; ++t)
+        if (ALL || !skip(t)) a = f(t, a);
+    }
+    a = row_sum16(a);
+    if constexpr (ROWS > 1) a = from_last(a);
+    return a;
+  }
+  template <class F>
+  FDT_DEV double chain_sum_d(F&& f) const {
+    double a = 0.0;
+#pragma unroll
+    for (int h = 0; h < ROWS; ++h) {
+      if (h) {
+        const int2 b = __builtin_bit_cast(int2, a);
+        a = __builtin_bit_cast(double, make_int2(__builtin_bit_cast(int, next_row(__builtin_bit_cast(float, b.x))),
+                                                 __builtin_bit_cast(int, next_row(__builtin_bit_cast(float, b.y)))));
+      }
+#pragma unroll
+      for (int t = 0; t < VPL; ++t) a = f(t, a);
+    }
+    a = row_sum16_d(a);
+    if constexpr (ROWS > 1) {
+      const int2 b = __builtin_bit_cast(int2, a);
+      a = __builtin_bit_cast(double, make_int2(__builtin_bit_cast(int, from_last(__builtin_bit_cast(float, b.x))),
+                                               __builtin_bit_cast(int, from_last(__builtin_bit_cast(float, b.y)))));
+    }
+    return a;
+  }
+  // Gaussian likelihood change when every residual moves by -c q(t); ALL: slot 0
+  // of b = 0 volumes too
+  template <bool ALL = false, class Q>
+  FDT_DEV float quad(Q&& q, float c) const {
+    if constexpr (ROWS == 1) {
+      Quad qd;
+#pragma unroll
+      for (int t = 0; t < VPL; ++t)
+        if (ALL || !skip(t)) qd.add(r[t], q(t));
+      return qd.delta(c);
+    } else {
+      float A = 0.0f, B = 0.0f;
+#pragma unroll
+      for (int h = 0; h < ROWS; ++h) {
+        if (h) { A = next_row(A); B = next_row(B); }
+#pragma unroll
+        for (int t = 0; t < VPL; ++t) { A = fmaf(r[t], q(t), A); B = fmaf(q(t), q(t), B); }
+      }
+      A = from_last(row_sum16(A));
+      B = from_last(row_sum16(B));
+      return c * fmaf(c, B, -2.0f * A);
+    }
+  }
   // options
   bool incf0, ardf0, can_ard;
   bool lam[K];
@@ -382,20 +462,17 @@ struct Chain {
 
   // rebuild M and the residual (or the Rician terms) from the stored signals
   FDT_DEV void rebuild(const float* y) {
-    double ss = 0.0;
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
       float m = mix(t);
       M[t] = m;
-      if constexpr (RIC) {
-        ell[t] = ell_of(yv(t), S0 * m, tau);
-        ss += (double)mask(t, ell[t]);
-      } else {
-        r[t] = mask(t, y[t] - S0 * m);
-        ss += (double)(r[t] * r[t]);
-      }
+      if constexpr (RIC) ell[t] = ell_of(yv(t), S0 * m, tau);
+      else r[t] = mask(t, y[t] - S0 * m);
     }
-    like = row_sum16_d(ss);
+    like = chain_sum_d([&](int t, double ss) {
+      if constexpr (RIC) return ss + (double)mask(t, ell[t]);
+      else return ss + (double)(r[t] * r[t]);
+    });
   }
 
   // ---------------------------------------------------------- proposals
@@ -435,16 +512,12 @@ struct Chain {
     const float fsn = fsum - f0 + f0n;
     if (f0n <= 0.0f || f0n >= 1.0f || fsn > 1.0f) return;
     const float df = f0n - f0;
-    float a = 0.0f, en[RIC ? VPL : 1], qv[VPL];
-    Quad qd;
+    float a, en[RIC ? VPL : 1], qv[VPL];
 #pragma unroll
-    for (int t = 0; t < VPL; ++t) {
-      if (skip(t)) continue;
-      qv[t] = 1.0f - isov(t);
-      if constexpr (!RIC) qd.add(r[t], qv[t]);
-    }
-    if constexpr (RIC) ric_terms<false>([&](int t) { return S0 * fmaf(df, qv[t], M[t]); }, tau, en, a);
-    a = RIC ? row_sum16(a) : qd.delta(S0 * df);
+    for (int t = 0; t < VPL; ++t)
+      if (!skip(t)) qv[t] = 1.0f - isov(t);
+    if constexpr (RIC) a = ric_terms<false>([&](int t) { return S0 * fmaf(df, qv[t], M[t]); }, tau, en);
+    else a = quad([&](int t) { return qv[t]; }, S0 * df);
     if (dlik(a) + dprior<SL_F0>() < -lu) {
       const float c = S0 * df;
 #pragma unroll
@@ -464,9 +537,8 @@ struct Chain {
     if constexpr (RIC) {
       const float tn = cand<SL_TAU>();
       if (tn <= 0.0f) return;
-      float a = 0.0f, en[VPL];
-      ric_terms<true>([&](int t) { return S0 * M[t]; }, tn, en, a);
-      a = row_sum16(a);  // change of the stored terms (the running sum's)
+      float en[VPL];
+      const float a = ric_terms<true>([&](int t) { return S0 * M[t]; }, tn, en);  // change of the stored terms
       // the -tau y^2 / 2 part of the full terms moves with tau too
       float dE = -Nf * (flog(tn) - flog(tau)) - fmaf(-0.5f * (tn - tau), yy, a);
       if (dE < -lu) {
@@ -483,14 +555,9 @@ struct Chain {
     const float Sn = cand<SL_S0>();
     if (Sn < 0.0f) return;
     const float dS = Sn - S0;
-    float a = 0.0f, en[RIC ? VPL : 1];
-    Quad qd;
-#pragma unroll
-    for (int t = 0; t < VPL; ++t) {
-      if constexpr (!RIC) qd.add(r[t], mask(t, M[t]));
-    }
-    if constexpr (RIC) ric_terms<true>([&](int t) { return Sn * M[t]; }, tau, en, a);
-    a = RIC ? row_sum16(a) : qd.delta(dS);
+    float a, en[RIC ? VPL : 1];
+    if constexpr (RIC) a = ric_terms<true>([&](int t) { return Sn * M[t]; }, tau, en);
+    else a = quad<true>([&](int t) { return mask(t, M[t]); }, dS);
     if (dlik(a) < -lu) {
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
@@ -525,8 +592,9 @@ struct Chain {
   static constexpr int RG = 3;
   // ALL: also slot 0 of b = 0 volumes (the S0 and tau moves).
   template <bool ALL, class P>
-  FDT_DEV void ric_terms(P&& p, float tv, float (&en)[RIC ? VPL : 1], float& a) const {
+  FDT_DEV float ric_terms(P&& p, float tv, float (&en)[RIC ? VPL : 1]) const {
     const float th = -0.5f * tv;
+    float a = 0.0f;
 #pragma unroll
     for (int t0 = 0; t0 < VPL; t0 += RG) {
       float q[RG], h[RG], x[RG];
@@ -556,9 +624,11 @@ struct Chain {
         const int t = t0 + i;
         if (out(t)) continue;
         en[t] = fmaf(h[i], q[i], x[i]);
-        a += mask(t, en[t] - ell[t]);
+        if constexpr (ROWS == 1) a += mask(t, en[t] - ell[t]);
       }
     }
+    if constexpr (ROWS == 1) return row_sum16(a);
+    else return chain_sum([&](int t, float z) { return z + mask(t, en[t] - ell[t]); });
   }
   // all stick signals and/or iso change: d (:924-985), d_std (:987-1051), R
   // (:1053-1122).  NA: the stick signals change, NI: the isotropic signal.
@@ -582,7 +652,8 @@ struct Chain {
     const SigC cn = aniso_coef<MODEL>(dn, dsn, Rn), ci = iso_coef<MODEL>(dn, dsn);
     fence();
     constexpr bool KEEP_M = U_LDS || RIC;
-    float a = 0.0f, mn[KEEP_M ? VPL : 1], en[RIC ? VPL : 1], sn[U_LDS ? K : 1][VPL];
+    constexpr bool KEEP_Q = !RIC && ROWS > 1;
+    float a, mn[KEEP_M ? VPL : 1], en[RIC ? VPL : 1], sn[U_LDS ? K : 1][VPL], qv[KEEP_Q ? VPL : 1];
     Dirs D;
     if constexpr (NA && !U_LDS) D = dirs();
     Quad qd;
@@ -628,15 +699,18 @@ struct Chain {
           }
           m = fmaf(fk[k], sk_, m);
         }
+        if (zero(t)) m = M[t];
         if constexpr (KEEP_M) mn[t] = m;
-        if constexpr (!RIC) qd.add(r[t], mask(t, m - M[t]));
+        if constexpr (KEEP_Q) qv[t] = mask(t, m - M[t]);
+        else if constexpr (!RIC) qd.add(r[t], mask(t, m - M[t]));
         // the gamma form has several temporaries per volume and signal: keep
         // the scheduler from overlapping many volumes of it (register spills)
         if constexpr ((NA && SA == 1) || (NI && SI == 1)) fence();
       }
     });
-    if constexpr (RIC) ric_terms<false>([&](int t) { return S0 * mn[t]; }, tau, en, a);
-    a = RIC ? row_sum16(a) : qd.delta(S0);
+    if constexpr (RIC) a = ric_terms<false>([&](int t) { return S0 * mn[t]; }, tau, en);
+    else if constexpr (KEEP_Q) a = quad([&](int t) { return qv[t]; }, S0);
+    else a = qd.delta(S0);
     if (dlik(a) + dprior<SL>() < -lu) {
       fence();
       by_shells<NI>([&](auto SHc) {
@@ -659,7 +733,7 @@ struct Chain {
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
         if (skip(t)) continue;
-        const float m = KEEP_M ? mn[KEEP_M ? t : 0] : mix(t);  // mix(t) repeats the candidate's expression
+        const float m = KEEP_M ? mn[KEEP_M ? t : 0] : (zero(t) ? M[t] : mix(t));  // mix(t) repeats the candidate's expression
         if constexpr (RIC) ell[t] = en[t]; else r[t] -= S0 * mask(t, m - M[t]);
         M[t] = m;
       }
@@ -683,7 +757,7 @@ struct Chain {
     xform(x0, x1, x2);
     fence();
     float sn[VPL], un[U_LDS ? VPL : 1], qv[VPL], en[RIC ? VPL : 1];
-    float a = 0.0f;
+    float a;
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
       if (skip(t)) continue;
@@ -693,15 +767,11 @@ struct Chain {
       if constexpr (U_LDS) un[t] = u;
       sn[t] = sig<STICK_KIND<MODEL>>(ca, u, bv(t, g));
     }
-    Quad qd;
 #pragma unroll
-    for (int t = 0; t < VPL; ++t) {
-      if (skip(t)) continue;
-      qv[t] = sn[t] - s[k][t];
-      if constexpr (!RIC) qd.add(r[t], qv[t]);
-    }
-    if constexpr (RIC) ric_terms<false>([&](int t) { return S0 * fmaf(fk[k], qv[t], M[t]); }, tau, en, a);
-    a = RIC ? row_sum16(a) : qd.delta(S0 * fk[k]);
+    for (int t = 0; t < VPL; ++t)
+      if (!skip(t)) qv[t] = sn[t] - s[k][t];
+    if constexpr (RIC) a = ric_terms<false>([&](int t) { return S0 * fmaf(fk[k], qv[t], M[t]); }, tau, en);
+    else a = quad([&](int t) { return qv[t]; }, S0 * fk[k]);
     if (dlik(a) + (IS_TH ? dprior<SL>() : 0.0f) < -lu) {
       const float c = S0 * fk[k];
 #pragma unroll
@@ -725,16 +795,12 @@ struct Chain {
     const float fsn = fsum - fk[k] + fn;
     if (fn <= 0.0f || fn >= 1.0f || fsn > 1.0f) return;
     const float df = fn - fk[k];
-    float a = 0.0f, en[RIC ? VPL : 1], qv[VPL];
-    Quad qd;
+    float a, en[RIC ? VPL : 1], qv[VPL];
 #pragma unroll
-    for (int t = 0; t < VPL; ++t) {
-      if (skip(t)) continue;
-      qv[t] = s[k][t] - isov(t);
-      if constexpr (!RIC) qd.add(r[t], qv[t]);
-    }
-    if constexpr (RIC) ric_terms<false>([&](int t) { return S0 * fmaf(df, qv[t], M[t]); }, tau, en, a);
-    a = RIC ? row_sum16(a) : qd.delta(S0 * df);
+    for (int t = 0; t < VPL; ++t)
+      if (!skip(t)) qv[t] = s[k][t] - isov(t);
+    if constexpr (RIC) a = ric_terms<false>([&](int t) { return S0 * fmaf(df, qv[t], M[t]); }, tau, en);
+    else a = quad([&](int t) { return qv[t]; }, S0 * df);
     if (dlik(a) + dprior<SL>() < -lu) {
       const float c = S0 * df;
 #pragma unroll
@@ -854,12 +920,16 @@ FDT_DEV bool zero_slot0(const ChainLds& L) {
 // :507-1474, run twice by CUDA/runmcmc.cu:108-316).  GN (--gradnonlin): the
 // chain reads its voxel's own corrected acquisition from a.acqv (the reference
 // indexes per-voxel bvals/alpha/beta with posBV, :266, :711).
-template <int K, int VPL, int MODEL, bool RIC, bool GN = false, bool FULL = false>
+template <int K, int VPL, int MODEL, bool RIC, bool GN = false, bool FULL = false, int ROWS = 1>
 FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
-  using C = Chain<K, VPL, MODEL, RIC, GN, FULL>;
+  using C = Chain<K, VPL, MODEL, RIC, GN, FULL, ROWS>;
+  static_assert(ROWS == 1 || (ROWS == 2 && !GN), "rows per voxel");
+  constexpr bool ZS = ZERO_SLOT<VPL * ROWS>;
   const int lane = __lane_id();
   const int rl = lane & 15;
-  const float4* sacq = L.acq;
+  const int h = ROWS > 1 ? (lane >> 4) % ROWS : 0;  // which of the voxel's rows
+  const int v0 = h * 16 * VPL;                       // its first volume
+  const float4* sacq = L.acq + v0;
   C c;
   c.rl = rl;
   c.acq = sacq;
@@ -869,7 +939,7 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
 #pragma unroll
     for (int t = 0; t < VPL; ++t) c.ga[t] = sacq[rl + 16 * t];
   }
-  c.sh = L.sh;
+  c.sh = GN ? nullptr : L.sh + v0;
   c.shb = L.shb;
   c.isot = GN ? L.iso : L.iso + (threadIdx.x >> 4) * 16;
   c.nshell = GN ? 0 : a.nshell;
@@ -878,7 +948,7 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
     float* bp = L.bp + (threadIdx.x >> 4) * (16 * VPL);
     float* gd = L.gd + (threadIdx.x >> 4) * 9;
     const float4* av = a.acqv + (size_t)vox * a.acqv_stride;
-    const int* pm = ZERO_SLOT<VPL> ? L.perm : nullptr;  // the staged order of the shared table
+    const int* pm = ZS ? L.perm : nullptr;  // the staged order of the shared table
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
       const int i = rl + 16 * t;
@@ -895,31 +965,34 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
   c.halfN = 0.5f * (float)a.N;
   c.Nf = (float)a.N;
   c.Rmean = a.Rmean; c.Rstd = a.Rstd; c.Rfudge = a.Rfudge;
-  c.nv = a.N > rl ? min(VPL, (a.N - rl + 15) >> 4) : 0;
+  c.nv = a.N - v0 > rl ? min(VPL, (a.N - v0 - rl + 15) >> 4) : 0;
 #pragma unroll
   for (int k = 0; k < K; ++k) c.lam[k] = (k == 0) ? (a.all_ard != 0) : (a.no_ard == 0);
 
   // ---- data (with the Rician non-positive replacement, CUDA/xfibres_gpu.cu:350-367)
   float y[VPL];
   const float* yrow = a.data + (size_t)vox * a.N;
-  const int* perm = ZERO_SLOT<VPL> ? L.perm : nullptr;  // volume of each slot position (null: identity)
-  c.z0 = zero_slot0<VPL>(L);
+  const int* perm = ZS ? L.perm : nullptr;  // volume of each slot position (null: identity)
+  c.z0 = zero_slot0<VPL * ROWS>(L) && h == 0;
 #pragma unroll
   for (int t = 0; t < VPL; ++t) {
-    int i = rl + 16 * t;
+    int i = v0 + rl + 16 * t;
     y[t] = i < a.N ? yrow[perm ? perm[i] : i] : 0.0f;
   }
   if (RIC) {
     float mn = 3.0e38f, mx = -3.0e38f, mnp = 3.0e38f;
 #pragma unroll
     for (int t = 0; t < VPL; ++t)
-      if (rl + 16 * t < a.N) { mn = fminf(mn, y[t]); mx = fmaxf(mx, y[t]); if (y[t] > 0.0f) mnp = fminf(mnp, y[t]); }
+      if (v0 + rl + 16 * t < a.N) { mn = fminf(mn, y[t]); mx = fmaxf(mx, y[t]); if (y[t] > 0.0f) mnp = fminf(mnp, y[t]); }
     mn = row_min16(mn); mx = row_max16(mx); mnp = row_min16(mnp);
+    if constexpr (ROWS > 1) {
+      mn = fminf(mn, __shfl_xor(mn, 16)); mx = fmaxf(mx, __shfl_xor(mx, 16)); mnp = fminf(mnp, __shfl_xor(mnp, 16));
+    }
     bool san = (mn <= 0.0f && mx > 0.0f);
 #pragma unroll
     for (int t = 0; t < VPL; ++t) {
       if (san && y[t] <= 0.0f) y[t] = mnp;
-      if (rl + 16 * t >= a.N) y[t] = 1.0f;
+      if (v0 + rl + 16 * t >= a.N) y[t] = 1.0f;
     }
   }
 
@@ -1015,10 +1088,7 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
       if constexpr (C::Y_LDS) c.vol[t * 64] = -2.0f * y[t];
       else c.r[t] = -2.0f * y[t];
     }
-    float yy = 0.0f;
-#pragma unroll
-    for (int t = 0; t < VPL; ++t) yy += c.mask(t, square(y[t]));
-    c.yy = row_sum16(yy);
+    c.yy = c.template chain_sum<true>([&](int t, float z) { return z + c.mask(t, square(y[t])); });
   }
   c.rebuild(y);
 
@@ -1036,6 +1106,7 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
     float* arr = w == 0 ? a.th : (w == 1 ? a.ph : a.f);
     if (arr) rec_base = arr + (size_t)k * a.nsamples * a.vstride;
   }
+  if (h) rec_base = nullptr;
   if (rec_base) rec_base += vox;
 
   const uint64_t gvox = a.vox_offset + (uint64_t)vox;
@@ -1082,7 +1153,7 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
         float yr[VPL];
 #pragma unroll
         for (int t = 0; t < VPL; ++t) {
-          const int i = rl + 16 * t;
+          const int i = v0 + rl + 16 * t;
           yr[t] = i < a.N ? yrow[perm ? perm[i] : i] : 0.0f;
         }
         c.rebuild(yr);
@@ -1093,34 +1164,30 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
     const float tau = c.tau;
     double e = c.like;
     if constexpr (RIC) {
-      double sl = 0.0, sy = 0.0;  // the model-independent part of the Rician terms
-#pragma unroll
-      for (int t = 0; t < VPL; ++t) {
+      // the model-independent part of the Rician terms
+      const double sl = c.chain_sum_d([&](int t, double z) { return z + (double)c.mask(t, flog(c.yv(t))); });
+      const double sy = c.chain_sum_d([&](int t, double z) {
         const double yd = (double)c.yv(t);
-        sl += (double)c.mask(t, flog(c.yv(t)));
-        sy += t < c.nv ? yd * yd : 0.0;
-      }
-      e = -(double)a.N * (double)flog(tau) - (c.like + row_sum16_d(sl) - 0.5 * (double)tau * row_sum16_d(sy));
+        return z + (t < c.nv ? yd * yd : 0.0);
+      });
+      e = -(double)a.N * (double)flog(tau) - (c.like + sl - 0.5 * (double)tau * sy);
     }
-    if (rl == 0) a.energy[vox] = (float)e;
+    if (rl == 0 && h == 0) a.energy[vox] = (float)e;
   }
   if (a.ssr) {  // sum of squares of the final state's residuals (the Rician chain keeps the data in r)
     double ss;
     if constexpr (RIC) {
       const float S0 = c.S0;
-      float acc = 0.0f;
-#pragma unroll
-      for (int t = 0; t < VPL; ++t) {
+      ss = (double)c.template chain_sum<true>([&](int t, float z) {
         const float e = c.yv(t) - S0 * c.M[t];
-        acc += c.mask(t, square(e));
-      }
-      ss = (double)row_sum16(acc);
+        return z + c.mask(t, square(e));
+      });
     } else {
       ss = c.like;
     }
-    if (rl == 0) a.ssr[vox] = (float)ss;
+    if (rl == 0 && h == 0) a.ssr[vox] = (float)ss;
   }
-  if (a.widths_out) a.widths_out[(size_t)vox * 16 + rl] = c.sprop;
+  if (a.widths_out && h == 0) a.widths_out[(size_t)vox * 16 + rl] = c.sprop;
 }
 
 

@@ -15,59 +15,99 @@ __device__ inline int xcd_tile(int b, int nb) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + l;
 }
 
-template <int K, int VPL, int MODEL, bool RIC, bool GN, bool FULL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VPL <= 18 ? 2 : 1, 2))) void mcmc_kernel(McmcArgs a) {
-  __shared__ float4 sacq[16 * VPL];
-  constexpr bool SMALL = Chain<K, VPL, MODEL, RIC, GN, FULL>::SMALL;  // state in registers
+// VPL volumes per lane in ROWS rows per voxel: a tile of VPL ROWS.
+template <int K, int VPL, int MODEL, bool RIC, bool GN, bool FULL, int ROWS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VPL <= 18 || (K == 1 && !RIC && !GN) ? 2 : 1, 2))) void mcmc_kernel(McmcArgs a) {
+  constexpr bool SMALL = Chain<K, VPL, MODEL, RIC, GN, FULL, ROWS>::SMALL;  // state in registers
+  constexpr int TILE = VPL * ROWS;
+  __shared__ float4 sacq[16 * TILE];
   __shared__ float sba[SMALL ? 1 : 4 * K * VPL * 64];
-  __shared__ int ssh[GN ? 1 : 16 * VPL];
+  __shared__ int ssh[GN ? 1 : 16 * TILE];
   __shared__ float sshb[16];
   __shared__ float siso[GN ? 1 : 16 * 16];
   __shared__ float sbp[GN ? 16 * 16 * VPL : 1];
   __shared__ float sgd[GN ? 16 * 9 : 1];
   __shared__ float svol[GN || SMALL ? 1 : 4 * VPL * 64];
-  constexpr bool ZS = ZERO_SLOT<VPL>;
-  __shared__ int sperm[ZS ? 16 * VPL : 1];
+  constexpr bool ZS = ZERO_SLOT<TILE>;
+  __shared__ int sperm[ZS ? 16 * TILE : 1];
   __shared__ int szc[ZS ? ZC_CHUNKS : 1];
   const ChainLds L{sacq, sba, GN ? nullptr : ssh, sshb, siso, sbp, sgd, GN ? nullptr : svol, ZS ? sperm : nullptr,
                    ZS ? szc : nullptr};
-  stage_acq<VPL>(a, L);
+  stage_acq<TILE>(a, L);
   __syncthreads();
-  const int i = xcd_tile(blockIdx.x, gridDim.x) * 16 + (threadIdx.x >> 4);
-  if (i < a.nvox) run_chain<K, VPL, MODEL, RIC, GN, FULL>(a, a.list ? a.list[i] : i, L);
+  const int i = xcd_tile(blockIdx.x, gridDim.x) * (16 / ROWS) + (threadIdx.x >> 4) / ROWS;
+  if (i < a.nvox) run_chain<K, VPL, MODEL, RIC, GN, FULL, ROWS>(a, a.list ? a.list[i] : i, L);
 }
 
 }  // namespace fdt
 
-// Two translation units per VPL value (-DFDT_VPL=...): -DFDT_MCMC_RIC=0 holds
-// the Gaussian kernels and the launcher, -DFDT_MCMC_RIC=1 the Rician ones
-// (built in parallel; each can take its own compiler options).  K = 1..3 and
-// models 1..3 (a kernel each: one that held all models at once took 128 KB of code at K = 3 and 98 scalar
-// registers more than there are), with the shared acquisition or per-voxel ones (--gradnonlin, a->acqv set; its stride must
-// cover 16 * VPL volumes).
+// Three translation units per tile FDT_VPL, built in parallel, each with its own
+// compiler options: -DFDT_MCMC_UNIT=0 holds the launcher and the Gaussian kernels
+// with one row per voxel, 1 the Rician ones, 2 the kernels with two rows (the
+// iterative scheduler of the others crashes on their row swap).  K = 1..3 and
+// models 1..3 have a kernel each (one that held all models at once took 128 KB of
+// code at K = 3 and 98 scalar registers more than there are), with the shared
+// acquisition or per-voxel ones (--gradnonlin, a->acqv set; its stride must cover
+// 16 * FDT_VPL volumes).
 #ifndef FDT_VPL
 #define FDT_VPL 18
 #endif
-#ifndef FDT_MCMC_RIC
-#define FDT_MCMC_RIC 0
+#ifndef FDT_MCMC_UNIT
+#define FDT_MCMC_UNIT 0
 #endif
 #define FDT_CAT2_(a, b) a##b
 #define FDT_CAT2(a, b) FDT_CAT2_(a, b)
 
+// Two rows per voxel (ms of 250 sweeps, one row -> two)
+// - for launches that one-row waves would leave on half of the 1,024 SIMDs or
+//   less, 64% of whose cycles then issue: up to 2,048 voxels Gaussian (288
+//   volumes, K=3, model 2: 2.73 -> 2.13 at 2,000 voxels, but 3,000 voxels 2.71 ->
+//   2.76), 4,096 Rician (8.39 -> 4.38 at 2,000, model 3);
+// - above 288 volumes, where one row takes more than half of a SIMD's registers
+//   and leaves it one wave: 24,000 voxels of 432 volumes, model 2: K=3 24.1 ->
+//   20.4, K=2 17.2 -> 15.2, Rician model 3 K=3 74.4 -> 48.8.  Gaussian chains of
+//   one fibre fit two waves of one row up to 448 volumes and stay there (7.9
+//   against 10.3).
+// At 288 volumes and 24,000 voxels one row is faster (K=3, model 2: 11.3 against
+// 15.1; Rician model 3 30.2 against 31.2): the second row repeats every
+// proposal's sums and decision.
+#define FDT_ONLY_TWO (FDT_VPL > 18)
+#define FDT_CAN_TWO (FDT_VPL % 2 == 0 && FDT_VPL >= 10)
+
 namespace {
+// tiles above 18 that keep a one-row kernel
+constexpr bool one_row_above(int K, bool rician) { return K == 1 && !rician && FDT_VPL <= 28; }
+#if FDT_MCMC_UNIT == 2
 template <int K, int MODEL, bool RIC>
 hipError_t launch_model(const fdt::McmcArgs* a, hipStream_t s) {
-  dim3 grid((a->nvox + 15) / 16), block(256);
+  const dim3 grid((a->nvox + 7) / 8), block(256);
+  hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL / 2, MODEL, RIC, false, false, 2>), grid, block, 0, s, *a);
+  return hipGetLastError();
+}
+#else
+template <int K, int MODEL, bool RIC>
+hipError_t launch_model(const fdt::McmcArgs* a, hipStream_t s) {
+  const dim3 grid((a->nvox + 15) / 16), block(256);
+  if (a->acqv) {
+    hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, true, false, 1>), grid, block, 0, s, *a);
+    return hipGetLastError();
+  }
+#if FDT_VPL == 18
   // 288 volumes (18 b = 0 and 270 directions) fill the 18-volume tile: a kernel without the padding masks there
   // (250,968 voxels, model 2: 1,013 -> 1,001 ms; model-3 Rician chains of 16,384 voxels, with the halved products
   // of their terms: 202 -> 185 ms)
-  constexpr bool CAN_FULL = FDT_VPL == 18;
-  if (a->acqv) hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, true, false>), grid, block, 0, s, *a);
-  else if (CAN_FULL && a->N == 16 * FDT_VPL)
-    hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false, CAN_FULL>), grid, block, 0, s, *a);
-  else hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false, false>), grid, block, 0, s, *a);
-  return hipGetLastError();
+  if (a->N == 16 * FDT_VPL) {
+    hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false, true, 1>), grid, block, 0, s, *a);
+    return hipGetLastError();
+  }
+#endif
+  if constexpr (!FDT_ONLY_TWO || one_row_above(K, RIC)) {
+    hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false, false, 1>), grid, block, 0, s, *a);
+    return hipGetLastError();
+  }
+  return hipErrorInvalidValue;
 }
+#endif
 template <int K, bool RIC>
 hipError_t launch_k(const fdt::McmcArgs* a, hipStream_t s) {
   if (a->model == 1) return launch_model<K, 1, RIC>(a, s);
@@ -84,15 +124,25 @@ hipError_t launch(const fdt::McmcArgs* a, int K, hipStream_t s) {
 }
 }  // namespace
 
-#if FDT_MCMC_RIC
+#if FDT_MCMC_UNIT == 2
+extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_two_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, int rician, hipStream_t s) {
+  return rician ? launch<true>(a, K, s) : launch<false>(a, K, s);
+}
+#elif FDT_MCMC_UNIT == 1
 extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, hipStream_t s) {
   return launch<true>(a, K, s);
 }
 #else
+extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_two_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, int rician, hipStream_t s);
 extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, hipStream_t s);
 extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, int rician, hipStream_t s) {
   if (a->nvox <= 0) return hipSuccess;
   if (a->acqv && a->acqv_stride < 16 * FDT_VPL) return hipErrorInvalidValue;
+#if FDT_CAN_TWO
+  const bool few = a->nvox <= (rician ? 4096 : 2048);
+  if (!a->acqv && (few || (FDT_ONLY_TWO && !one_row_above(K, rician))))
+    return FDT_CAT2(fdt_launch_mcmc_two_vpl, FDT_VPL)(a, K, rician, s);
+#endif
   return rician ? FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(a, K, s) : launch<false>(a, K, s);
 }
 #endif

@@ -70,7 +70,7 @@ extern "C" {
 hipError_t fdt_launch_finish(const FinishArgs*, hipStream_t);
 #define FDT_NA_VPL(V) hipError_t fdt_launch_mcmc_vpl##V(const McmcArgs*, int, int, hipStream_t);
 FDT_NA_VPL(3) FDT_NA_VPL(5) FDT_NA_VPL(7) FDT_NA_VPL(10) FDT_NA_VPL(14) FDT_NA_VPL(18) FDT_NA_VPL(24)
-FDT_NA_VPL(27) FDT_NA_VPL(32)
+FDT_NA_VPL(28) FDT_NA_VPL(32)
 #undef FDT_NA_VPL
 
 int fdt_mcmc_noalloc(const fdt_opts* o, int N, const float* d_bvals, const float* d_bvecs, const float* d_data,
@@ -98,7 +98,7 @@ int fdt_mcmc_noalloc(const fdt_opts* o, int N, const float* d_bvals, const float
   struct Tile { int vpl; hipError_t (*fn)(const McmcArgs*, int, int, hipStream_t); };
   const Tile tiles[] = {{3, fdt_launch_mcmc_vpl3},   {5, fdt_launch_mcmc_vpl5},   {7, fdt_launch_mcmc_vpl7},
                         {10, fdt_launch_mcmc_vpl10}, {14, fdt_launch_mcmc_vpl14}, {18, fdt_launch_mcmc_vpl18},
-                        {24, fdt_launch_mcmc_vpl24}, {27, fdt_launch_mcmc_vpl27}, {32, fdt_launch_mcmc_vpl32}};
+                        {24, fdt_launch_mcmc_vpl24}, {28, fdt_launch_mcmc_vpl28}, {32, fdt_launch_mcmc_vpl32}};
   const Tile* tile = nullptr;
   for (const auto& t : tiles)
     if (16 * t.vpl >= N) { tile = &t; break; }
