@@ -1113,7 +1113,7 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
   const int total = a.nburn + a.njumps;
   for (int j = 0; j < total; ++j) {
     float nl, lul;
-    draw(a.seed, gvox, (uint32_t)j, (uint32_t)rl, nl, lul);
+    draw<!RIC>(a.seed, gvox, (uint32_t)j, (uint32_t)rl, nl, lul);
     c.propose(nl);
     if (c.incf0) c.prop_f0(row_bcast<SL_F0>(lul));
     if (RIC) c.prop_tau(row_bcast<SL_TAU>(lul));

@@ -143,17 +143,30 @@ FDT_DEV double uni(double v) {
 // ----------------------------------------------------------------- Philox
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11).  Draw layout:
 // key = (lo32 seed, hi32 seed), counter = (lo32 voxel, hi32 voxel, jump, slot).
+// PAIR: both halves of a product from one v_mad_u64_u32 and the two xors from
+// one v_bitop3_b32, 36 instructions fewer than v_mul_lo/v_mul_hi and v_xor (1,366
+// for 1,402 in the kernel of two fibres at 80 volumes).  A run of 250,968 voxels
+// at 288 volumes and three fibres: 1,270 -> 1,262 ms; the wavefronts over 1,440
+// voxels at 69 volumes: 243 -> 237.5 ms.  The Rician kernel has no registers left for the
+// pairs (185 -> 189 ms for 16,384 voxels at 288 volumes) and keeps the halves.
 struct u4 { uint32_t x, y, z, w; };
+template <bool PAIR>
 FDT_DEV u4 philox4x32_10(u4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
-    uint32_t hi0 = __umulhi(0xD2511F53u, c.x), lo0 = 0xD2511F53u * c.x;
-    uint32_t hi1 = __umulhi(0xCD9E8D57u, c.z), lo1 = 0xCD9E8D57u * c.z;
     u4 n;
-    n.x = hi1 ^ c.y ^ k0;
-    n.y = lo1;
-    n.z = hi0 ^ c.w ^ k1;
-    n.w = lo0;
+    if constexpr (PAIR) {
+      const uint64_t p0 = (uint64_t)0xD2511F53u * c.x, p1 = (uint64_t)0xCD9E8D57u * c.z;
+      n.x = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c.y, k0, 0x96);
+      n.y = (uint32_t)p1;
+      n.z = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c.w, k1, 0x96);
+      n.w = (uint32_t)p0;
+    } else {
+      n.x = __umulhi(0xCD9E8D57u, c.z) ^ c.y ^ k0;
+      n.y = 0xCD9E8D57u * c.z;
+      n.z = __umulhi(0xD2511F53u, c.x) ^ c.w ^ k1;
+      n.w = 0xD2511F53u * c.x;
+    }
     c = n;
     k0 += 0x9E3779B9u;
     k1 += 0xBB67AE85u;
@@ -167,9 +180,10 @@ FDT_DEV u4 philox4x32_10(u4 c, uint32_t k0, uint32_t k1) {
 // within 7.6e-7 of the double-precision mapping and log u within 1.7e-7
 // relative, over all 2^24 values of u2 (libm's float forms: 1.7e-6, from
 // rounding 2 pi u2 before the cosine).
+template <bool PAIR>
 FDT_DEV void draw(uint64_t seed, uint64_t vox, uint32_t jump, uint32_t slot, float& n, float& logu) {
   u4 c{(uint32_t)vox, (uint32_t)(vox >> 32), jump, slot};
-  u4 x = philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+  u4 x = philox4x32_10<PAIR>(c, (uint32_t)seed, (uint32_t)(seed >> 32));
   const float s24 = 1.0f / 16777216.0f, LN2 = 0.69314718055994531f;
   float u1 = (float)((x.x >> 8) + 1u) * s24;
   float u2 = (float)(x.y >> 8) * s24;
