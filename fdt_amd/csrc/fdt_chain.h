@@ -181,7 +181,10 @@ FDT_DEV float square(float x) {
 #pragma clang fp contract(off)
   return x * x;
 }
-
+FDT_DEV float product(float x, float y) {
+#pragma clang fp contract(off)
+  return x * y;
+}
 
 // One chain per 16-lane row.  Volume state lives in registers per lane;
 // everything that belongs to a proposal slot -- the parameter value, its
@@ -256,6 +259,8 @@ struct Chain {
   // slot 0 holds b = 0 volumes only (see stage_acq): the moves that leave
   // their signals at 1 skip it (ZERO_SLOT tiles only)
   bool z0;
+  bool th;   // a theta slot's lane
+  float pw;  // weight of the slot's log prior (see prior_weight)
   FDT_DEV bool skip(int t) const { return ROWS == 1 && ZERO_SLOT<VPL> && t == 0 && z0; }
   // two rows: this lane's slot t is in the slot of b = 0 volumes
   FDT_DEV bool zero(int t) const { return ROWS > 1 && ZERO_SLOT<VPL * ROWS> && t == 0 && z0; }
@@ -475,6 +480,22 @@ struct Chain {
     });
   }
 
+  // The prior energy of a slot is pw log(x), x the candidate or, for a theta
+  // slot, half the size of its sine: one weight per lane, fixed before the
+  // first sweep.  Asking which slot a lane is, and two remainders for the sweep
+  // numbers, cost about 50 scalar instructions and six branches per sweep, which
+  // the other waves of a SIMD do not hide and a single one waits for: 237.5 ->
+  // 215.6 ms for the wavefronts over 1,440 voxels at 69 volumes, 1,262 -> 1,242 ms
+  // for a run of 250,968 voxels at 288.
+  FDT_DEV void prior_weight() {
+    th = rl >= SL_FIB && (rl - SL_FIB) % 3 == 0;
+    pw = th ? -1.0f : 0.0f;
+    if (rl == SL_DSTD || (rl == SL_F0 && ardf0)) pw = 1.0f;
+    sfor<K>([&](auto kc) {
+      if (rl == FK(kc) && can_ard && lam[kc]) pw = fudge;
+    });
+  }
+
   // ---------------------------------------------------------- proposals
   // The candidates of every slot from the sweep's normal draws, lane l for
   // slot l (the R slot's prior depends on d and is formed at its proposal).
@@ -482,16 +503,10 @@ struct Chain {
   FDT_DEV void propose(float n) {
     sxn = sval + n * sprop;
     sincos_full(sxn, ssn, scn);
-    const bool th = rl >= SL_FIB && (rl - SL_FIB) % 3 == 0;
     const float lg = lg2(th ? fabsf(ssn) * 0.5f : sxn);
     const float L = lg * LN2;
-    float p = 0.0f;
-    if (th) p = sxn == 0.0f ? 0.0f : -L;
+    float p = pw == 0.0f || (th && sxn == 0.0f) ? 0.0f : product(pw, L);
     if (MODEL == 3 && rl == SL_D) p = fmaf(sxn, 4000.0f, -(L + L));
-    if (rl == SL_DSTD || (rl == SL_F0 && ardf0)) p = L;
-    sfor<K>([&](auto kc) {
-      if (rl == FK(kc) && can_ard && lam[kc]) p = fudge * L;
-    });
     sprn = p;
     sdp = rl == SL_DSTD ? fmaf(lg, LN2, -sprior) : p - sprior;
     accm = 0;
@@ -1111,6 +1126,10 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
 
   const uint64_t gvox = a.vox_offset + (uint64_t)vox;
   const int total = a.nburn + a.njumps;
+  c.prior_weight();
+  // sweeps to the next record and to the next change of the widths (counted
+  // down: see prior_weight)
+  int to_record = a.se, to_widths = a.upe, smp = 0;
   for (int j = 0; j < total; ++j) {
     float nl, lul;
     draw<!RIC>(a.seed, gvox, (uint32_t)j, (uint32_t)rl, nl, lul);
@@ -1134,14 +1153,13 @@ FDT_DEV void run_chain(const McmcArgs& a, int vox, const ChainLds& L) {
     c.settle();
 
     // record: the lane of each sampled slot writes its value
-    if (j >= a.nburn) {
-      int rec = j - a.nburn + 1;
-      if (a.se > 0 && rec % a.se == 0) {
-        int smp = rec / a.se - 1;
-        if (smp < a.nsamples && rec_base) rec_base[(size_t)smp * rec_stride] = c.sval;
-      }
+    if (a.se > 0 && j >= a.nburn && --to_record == 0) {
+      to_record = a.se;
+      if (smp < a.nsamples && rec_base) rec_base[(size_t)smp * rec_stride] = c.sval;
+      ++smp;
     }
-    if ((j + 1) % a.upe == 0) {
+    if (--to_widths == 0) {
+      to_widths = a.upe;
       c.update_proposals();
       // Re-anchor the incremental state with the widths: the mixtures, the
       // residuals (Gaussian: from the data, re-read) and the running

@@ -147,8 +147,9 @@ FDT_DEV double uni(double v) {
 // one v_bitop3_b32, 36 instructions fewer than v_mul_lo/v_mul_hi and v_xor (1,366
 // for 1,402 in the kernel of two fibres at 80 volumes).  A run of 250,968 voxels
 // at 288 volumes and three fibres: 1,270 -> 1,262 ms; the wavefronts over 1,440
-// voxels at 69 volumes: 243 -> 237.5 ms.  The Rician kernel has no registers left for the
-// pairs (185 -> 189 ms for 16,384 voxels at 288 volumes) and keeps the halves.
+// voxels at 69 volumes: 243 -> 237.5 ms.  The Rician kernel has no registers left
+// for the pairs (185 -> 189 ms for 16,384 voxels at 288 volumes) and keeps the
+// halves.
 struct u4 { uint32_t x, y, z, w; };
 template <bool PAIR>
 FDT_DEV u4 philox4x32_10(u4 c, uint32_t k0, uint32_t k1) {
@@ -173,6 +174,17 @@ FDT_DEV u4 philox4x32_10(u4 c, uint32_t k0, uint32_t k1) {
   }
   return c;
 }
+// sqrtf of zero or of a number far from the ends of its range: the hardware's
+// root, within one ulp, moved to the neighbour on whose side of the midpoint x
+// lies.  sqrtf also scales tiny arguments and tests for infinities, seven
+// instructions more; -2 log u is 0 or in [1.1e-7, 33.3].
+FDT_DEV float sqrt_nearest(float x) {
+  const float s = __builtin_amdgcn_sqrtf(x);
+  const float lo = __builtin_bit_cast(float, __builtin_bit_cast(int, s) - 1);
+  const float hi = __builtin_bit_cast(float, __builtin_bit_cast(int, s) + 1);
+  float r = fmaf(-lo, s, x) <= 0.0f ? lo : s;
+  return fmaf(-hi, s, x) > 0.0f ? hi : r;
+}
 // Standard normal by Box-Muller (cosine branch) and log of an acceptance
 // uniform in (0,1], from one Philox block (24-bit uniforms).  With the
 // hardware log2 and cos (v_cos_f32 takes its argument in revolutions, so
@@ -188,7 +200,7 @@ FDT_DEV void draw(uint64_t seed, uint64_t vox, uint32_t jump, uint32_t slot, flo
   float u1 = (float)((x.x >> 8) + 1u) * s24;
   float u2 = (float)(x.y >> 8) * s24;
   float u3 = (float)((x.z >> 8) + 1u) * s24;
-  n = sqrtf(-2.0f * LN2 * __builtin_amdgcn_logf(u1)) * __builtin_amdgcn_cosf(u2);
+  n = sqrt_nearest(-2.0f * LN2 * __builtin_amdgcn_logf(u1)) * __builtin_amdgcn_cosf(u2);
   logu = LN2 * __builtin_amdgcn_logf(u3);
 }
 
