@@ -72,8 +72,8 @@ namespace {
 typedef hipError_t (*mcmc_launch_fn)(const McmcArgs*, int, int, hipStream_t);
 struct VplEntry { int vpl; mcmc_launch_fn fn; };
 // In steps of about a third, so that little of a tile is padding: with 3, 5, 10, 18, 24 and 32 alone the chains of
-// 432 volumes ran in 32 slots instead of 27 (3,001 voxels, model 2, K = 2, --f0: 68.0 -> 61.0 ms with the fit), those
-// of 200 volumes in 18 instead of 14
+// 432 volumes ran in 32 slots instead of 28 (3,001 voxels, model 2, K = 2, --f0: 68.0 -> 61.0 ms with the fit; 53 in
+// two rows of 14), those of 200 volumes in 18 instead of 14
 const VplEntry kVpl[] = {{3, fdt_launch_mcmc_vpl3},   {5, fdt_launch_mcmc_vpl5},   {7, fdt_launch_mcmc_vpl7},
                          {10, fdt_launch_mcmc_vpl10}, {14, fdt_launch_mcmc_vpl14}, {18, fdt_launch_mcmc_vpl18},
                          {24, fdt_launch_mcmc_vpl24}, {28, fdt_launch_mcmc_vpl28}, {32, fdt_launch_mcmc_vpl32}};

@@ -19,8 +19,10 @@
 // sweep: evaluating what belongs to a slot once per sweep in its own lane,
 // keeping the stick arguments for the diffusivity moves and each proposal's
 // per-volume changes for its acceptance took 5,107 VALU instructions per wave
-// and sweep to 4,193, and one kernel per model (128 KB of code to 54, no
-// spilled vector registers) let the launch follow: 1,247 to 1,020 ms.
+// and sweep to 4,154, and one kernel per model (128 KB of code to 54, no
+// spilled vector registers) let the launch follow: 1,247 to 1,013 ms.  Masks
+// compiled out at 288 volumes, the draws' products from one instruction and no
+// question about a slot or a sweep number inside a sweep: 973 ms.
 // A proposal evaluates only what it changes; its likelihood change is
 // summed over the row with DPP adds.  For Gaussian noise a move of every
 // residual by -c*q gives the change of the sum of squares c*(c*sum q^2 -
@@ -68,8 +70,8 @@ enum { SL_F0 = 0, SL_TAU = 1, SL_D = 2, SL_DSTD = 3, SL_R = 4, SL_S0 = 5, SL_FIB
 // stage_acq): the 14- and 18-volume tiles, where it saves 3-4% of the chain time.  In
 // the smaller tiles the uniform branch around slot 0 costs more than it saves
 // (it splits the few volumes a lane interleaves); at 24 and 32 volumes per
-// lane (one wave per SIMD) it saved nothing (N = 384 with 24 b = 0 volumes)
-// and cost 1.4% (N = 432).
+// lane in one row (one wave per SIMD) it saved nothing (N = 384 with 24 b = 0
+// volumes) and cost 1.4% (N = 432).
 template <int VPL> constexpr bool ZERO_SLOT = VPL == 14 || VPL == 18;
 
 // Signal forms with row-uniform coefficients (compute_signal /
@@ -213,7 +215,7 @@ struct Chain {
   // Tiles of up to 5 volumes per lane keep everything in registers, the
   // acquisition and the stick arguments too: their proposals are short chains
   // of dependent operations, where each LDS read adds its latency (2,000
-  // voxels of 69 volumes, model 1: 5.5 -> 4.4 ms).  At 10 volumes per lane and
+  // voxels of 69 volumes, model 1: 5.5 -> 4.5 ms).  At 10 volumes per lane and
   // K=3 the registers run out (48 spilled).
   static constexpr bool SMALL = VPL <= 5;
   static constexpr bool ISO_LDS = !GN && !RIC && !SMALL, Y_LDS = !GN && RIC && !SMALL;
@@ -266,7 +268,7 @@ struct Chain {
   FDT_DEV bool zero(int t) const { return ROWS > 1 && ZERO_SLOT<VPL * ROWS> && t == 0 && z0; }
   // A running sum handed from the first row to the second (0 to the first): the
   // gfx950 row swap exchanges the odd rows of its first operand with the even
-  // rows of its second; clang 20 gives the first result for the second one too,
+  // rows of its second; clang 22 gives the first result for the second one too,
   // so only the first is used.
   static FDT_DEV float next_row(float a) {
     const auto w = __builtin_amdgcn_permlane16_swap(0, __builtin_bit_cast(int, a), false, false);
@@ -480,6 +482,12 @@ struct Chain {
     });
   }
 
+  // A candidate out of its range is refused with the energy's own test: a
+  // branch of its own saves the evaluation only where all four rows of a wave
+  // are out of range at once (the wavefronts over 1,440 voxels at 69 volumes:
+  // 215.6 -> 210.3 ms without it).  The Rician terms are dear enough to keep it.
+  static constexpr bool EARLY = RIC;
+
   // The prior energy of a slot is pw log(x), x the candidate or, for a theta
   // slot, half the size of its sine: one weight per lane, fixed before the
   // first sweep.  Asking which slot a lane is, and two remainders for the sweep
@@ -525,7 +533,8 @@ struct Chain {
   FDT_DEV void prop_f0(float lu) {
     const float f0n = cand<SL_F0>();
     const float fsn = fsum - f0 + f0n;
-    if (f0n <= 0.0f || f0n >= 1.0f || fsn > 1.0f) return;
+    const bool in = !(f0n <= 0.0f || f0n >= 1.0f || fsn > 1.0f);
+    if (EARLY && !in) return;
     const float df = f0n - f0;
     float a, en[RIC ? VPL : 1], qv[VPL];
 #pragma unroll
@@ -533,7 +542,7 @@ struct Chain {
       if (!skip(t)) qv[t] = 1.0f - isov(t);
     if constexpr (RIC) a = ric_terms<false>([&](int t) { return S0 * fmaf(df, qv[t], M[t]); }, tau, en);
     else a = quad([&](int t) { return qv[t]; }, S0 * df);
-    if (dlik(a) + dprior<SL_F0>() < -lu) {
+    if (in & (dlik(a) + dprior<SL_F0>() < -lu)) {
       const float c = S0 * df;
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
@@ -568,12 +577,13 @@ struct Chain {
   // S0 (:1125-1155)
   FDT_DEV void prop_S0(float lu) {
     const float Sn = cand<SL_S0>();
-    if (Sn < 0.0f) return;
+    const bool in = !(Sn < 0.0f);
+    if (EARLY && !in) return;
     const float dS = Sn - S0;
     float a, en[RIC ? VPL : 1];
     if constexpr (RIC) a = ric_terms<true>([&](int t) { return Sn * M[t]; }, tau, en);
     else a = quad<true>([&](int t) { return mask(t, M[t]); }, dS);
-    if (dlik(a) < -lu) {
+    if (in & (dlik(a) < -lu)) {
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
         if constexpr (RIC) ell[t] = en[t]; else r[t] -= dS * mask(t, M[t]);
@@ -652,18 +662,20 @@ struct Chain {
     constexpr bool NA = !(SL == SL_DSTD && MODEL == 3), NI = SL != SL_R;
     constexpr int SA = STICK_KIND<MODEL>, SI = ISO_KIND<MODEL>;
     float dn = d, dsn = dstd, Rn = Rr;
+    bool in;
     if constexpr (SL == SL_D) {
       dn = cand<SL>();
-      if (dn < 0.0f || dn > UPPERDIFF_F) return;
+      in = !(dn < 0.0f || dn > UPPERDIFF_F);
     } else if constexpr (SL == SL_DSTD) {
       dsn = cand<SL>();
-      if (dsn <= 0.0f || dsn > (MODEL == 3 ? 0.004f : 0.01f)) return;
+      in = !(dsn <= 0.0f || dsn > (MODEL == 3 ? 0.004f : 0.01f));
     } else {
       Rn = cand<SL>();
       float prn = 0.0f;
-      if (!r_prior(Rn, d, prn)) return;
-      if (rl == SL_R) { sprn = prn; sdp = prn - sprior; }
+      in = r_prior(Rn, d, prn);
+      if (rl == SL_R && in) { sprn = prn; sdp = prn - sprior; }
     }
+    if (EARLY && !in) return;
     const SigC cn = aniso_coef<MODEL>(dn, dsn, Rn), ci = iso_coef<MODEL>(dn, dsn);
     fence();
     constexpr bool KEEP_M = U_LDS || RIC;
@@ -726,7 +738,7 @@ struct Chain {
     if constexpr (RIC) a = ric_terms<false>([&](int t) { return S0 * mn[t]; }, tau, en);
     else if constexpr (KEEP_Q) a = quad([&](int t) { return qv[t]; }, S0);
     else a = qd.delta(S0);
-    if (dlik(a) + dprior<SL>() < -lu) {
+    if (in & (dlik(a) + dprior<SL>() < -lu)) {
       fence();
       by_shells<NI>([&](auto SHc) {
 #pragma unroll
@@ -808,7 +820,8 @@ struct Chain {
     constexpr int SL = FK(k);
     const float fn = cand<SL>();
     const float fsn = fsum - fk[k] + fn;
-    if (fn <= 0.0f || fn >= 1.0f || fsn > 1.0f) return;
+    const bool in = !(fn <= 0.0f || fn >= 1.0f || fsn > 1.0f);
+    if (EARLY && !in) return;
     const float df = fn - fk[k];
     float a, en[RIC ? VPL : 1], qv[VPL];
 #pragma unroll
@@ -816,7 +829,7 @@ struct Chain {
       if (!skip(t)) qv[t] = s[k][t] - isov(t);
     if constexpr (RIC) a = ric_terms<false>([&](int t) { return S0 * fmaf(df, qv[t], M[t]); }, tau, en);
     else a = quad([&](int t) { return qv[t]; }, S0 * df);
-    if (dlik(a) + dprior<SL>() < -lu) {
+    if (in & (dlik(a) + dprior<SL>() < -lu)) {
       const float c = S0 * df;
 #pragma unroll
       for (int t = 0; t < VPL; ++t) {
