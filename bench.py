@@ -29,10 +29,10 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, HERE)
 
 FP32_PEAK_TFLOPS = 157.3
-# HBM bytes per launch of mcmc_kernel<3,18,2,false,false> on the full 250,968-voxel
+# HBM bytes per launch of mcmc_kernel<3,18,2,false,false,true,1> on the full 250,968-voxel
 # workload: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE, each scaled by the same
 # counter's reading for a copy kernel of known size (profiles/mcmc_c1_traffic.md)
-MCMC_TRAFFIC_BYTES = (2 * 148124 + 632652) * 1024
+MCMC_TRAFFIC_BYTES = (2 * 147477 + 617261) * 1024
 METRIC = "voxels/s, 3-fibre multi-shell bedpostx; surrogate vs plain at equal dyad error"
 LM_MODES = {0: "FP32 model, Jacobian and cost", 1: "FP64 throughout",
             2: "FP32 Jacobian and normal equations, FP64 parameters and cost"}
@@ -382,7 +382,7 @@ def bench_gradnonlin(args):
                                "gradient deviations (grad_dev ~ N(0, 0.03)), --gradnonlin, bi=1000 nj=1250 se=25",
                    "ms_fit": g["ms_fit"], "ms_mcmc": g["ms_mcmc"], "s_synth": t_syn},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / FP32_PEAK_TFLOPS, "traffic": None, "kernel": "mcmc_kernel<3,18,false,true>",
+                     "frac": achieved / FP32_PEAK_TFLOPS, "traffic": None, "kernel": "mcmc_kernel<3,18,2,false,true,false,1>",
                      "flops_per_launch": fl_launch},
         "shared_acquisition": {"voxels_per_s": p["rate"], "ms_fit": p["ms_fit"], "ms_mcmc": p["ms_mcmc"]},
         "dyad_err_median_deg": {"gradnonlin": g["dyad"], "deviations_ignored": p["dyad"]},
@@ -753,7 +753,7 @@ def main():
                    "mcmc_tile": f"{tm['lanes']} lanes x {tm['vpl']} volumes per voxel"},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP32_PEAK_TFLOPS, "traffic": traffic,
-                     "kernel": "mcmc_kernel<3,18,2,false,false>", "flops_per_launch": fl_launch,
+                     "kernel": "mcmc_kernel<3,18,2,false,false,true,1>", "flops_per_launch": fl_launch,
                      "compute": "FP32 vector ALU (no matrix-shaped work on this path); peak is the published "
                                 "FP32 figure, which counts packed FP32 -- this build disables packed FP32, so "
                                 "half of it (78.6) is the reachable issue ceiling"},
