@@ -48,14 +48,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES<K, VP
 
 }  // namespace fdt
 
-// Three translation units per tile FDT_VPL, built in parallel, each with its own
-// compiler options: -DFDT_MCMC_UNIT=0 holds the launcher and the Gaussian kernels
-// with one row per voxel, 1 the Rician ones, 2 the kernels with two rows (the
-// iterative scheduler of the others crashes on their row swap).  K = 1..3 and
-// models 1..3 have a kernel each (one that held all models at once took 128 KB of
-// code at K = 3 and 98 scalar registers more than there are), with the shared
-// acquisition or per-voxel ones (--gradnonlin, a->acqv set; its stride must cover
-// 16 * FDT_VPL volumes).
+// Up to six translation units per tile FDT_VPL, built in parallel, each with its
+// own compiler options and loaded with its first launch: -DFDT_MCMC_UNIT=0 holds
+// the launcher and the Gaussian kernels with one row per voxel, 1 the Rician
+// ones, 2 the kernels with two rows (the iterative scheduler of the others
+// crashes on their row swap); 3, 4 and 5 are 0, 1 and 2 for acquisitions that
+// fill the tile.  K = 1..3 and models 1..3 have a kernel each (one that held all
+// models at once took 128 KB of code at K = 3 and 98 scalar registers more than
+// there are), with the shared acquisition or per-voxel ones (--gradnonlin,
+// a->acqv set; its stride must cover 16 * FDT_VPL volumes; units 0 and 1).
 #ifndef FDT_VPL
 #define FDT_VPL 18
 #endif
@@ -82,39 +83,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES<K, VP
 #define FDT_CAN_TWO (FDT_VPL % 2 == 0 && FDT_VPL >= 10)
 
 namespace {
+constexpr bool FULL = FDT_MCMC_UNIT >= 3;
+constexpr int ROWS = FDT_MCMC_UNIT % 3 == 2 ? 2 : 1;
 // tiles above 18 that keep a one-row kernel
 constexpr bool one_row_above(int K, bool rician) { return K == 1 && !rician && FDT_VPL <= 28; }
-#if FDT_MCMC_UNIT == 2
 template <int K, int MODEL, bool RIC>
 hipError_t launch_model(const fdt::McmcArgs* a, hipStream_t s) {
-  const dim3 grid((a->nvox + 7) / 8), block(256);
-  hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL / 2, MODEL, RIC, false, false, 2>), grid, block, 0, s, *a);
-  return hipGetLastError();
-}
-#else
-template <int K, int MODEL, bool RIC>
-hipError_t launch_model(const fdt::McmcArgs* a, hipStream_t s) {
-  const dim3 grid((a->nvox + 15) / 16), block(256);
-  if (a->acqv) {
-    hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, true, false, 1>), grid, block, 0, s, *a);
-    return hipGetLastError();
+  const dim3 grid((a->nvox + 16 / ROWS - 1) / (16 / ROWS)), block(256);
+  if constexpr (!FULL && ROWS == 1) {
+    if (a->acqv) {
+      hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, true, false, 1>), grid, block, 0, s, *a);
+      return hipGetLastError();
+    }
   }
-#if FDT_VPL == 18
-  // 288 volumes (18 b = 0 and 270 directions) fill the 18-volume tile: a kernel without the padding masks there
-  // (250,968 voxels, model 2: 1,013 -> 1,001 ms; model-3 Rician chains of 16,384 voxels, with the halved products
-  // of their terms: 202 -> 185 ms)
-  if (a->N == 16 * FDT_VPL) {
-    hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false, true, 1>), grid, block, 0, s, *a);
-    return hipGetLastError();
-  }
-#endif
-  if constexpr (!FDT_ONLY_TWO || one_row_above(K, RIC)) {
-    hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL, MODEL, RIC, false, false, 1>), grid, block, 0, s, *a);
+  if constexpr (ROWS == 2 || !FDT_ONLY_TWO || one_row_above(K, RIC)) {
+    hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL / ROWS, MODEL, RIC, false, FULL, ROWS>), grid, block, 0, s, *a);
     return hipGetLastError();
   }
   return hipErrorInvalidValue;
 }
-#endif
 template <int K, bool RIC>
 hipError_t launch_k(const fdt::McmcArgs* a, hipStream_t s) {
   if (a->model == 1) return launch_model<K, 1, RIC>(a, s);
@@ -131,25 +118,47 @@ hipError_t launch(const fdt::McmcArgs* a, int K, hipStream_t s) {
 }
 }  // namespace
 
-#if FDT_MCMC_UNIT == 2
-extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_two_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, int rician, hipStream_t s) {
-  return rician ? launch<true>(a, K, s) : launch<false>(a, K, s);
-}
-#elif FDT_MCMC_UNIT == 1
-extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, hipStream_t s) {
+#define FDT_UNIT(u) FDT_CAT2(FDT_CAT2(FDT_CAT2(fdt_launch_mcmc_unit, u), _vpl), FDT_VPL)
+#define FDT_UNIT_ARGS (const fdt::McmcArgs* a, int K, int rician, hipStream_t s)
+extern "C" {
+#if FDT_MCMC_UNIT
+hipError_t FDT_UNIT(FDT_MCMC_UNIT) FDT_UNIT_ARGS {
+#if FDT_MCMC_UNIT == 1 || FDT_MCMC_UNIT == 4
   return launch<true>(a, K, s);
+#elif FDT_MCMC_UNIT == 3
+  return launch<false>(a, K, s);
+#else
+  return rician ? launch<true>(a, K, s) : launch<false>(a, K, s);
+#endif
 }
 #else
-extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_two_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, int rician, hipStream_t s);
-extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, hipStream_t s);
-extern "C" hipError_t FDT_CAT2(fdt_launch_mcmc_vpl, FDT_VPL)(const fdt::McmcArgs* a, int K, int rician, hipStream_t s) {
+hipError_t FDT_UNIT(1) FDT_UNIT_ARGS;
+hipError_t FDT_UNIT(2) FDT_UNIT_ARGS;
+hipError_t FDT_UNIT(3) FDT_UNIT_ARGS;
+hipError_t FDT_UNIT(4) FDT_UNIT_ARGS;
+hipError_t FDT_UNIT(5) FDT_UNIT_ARGS;
+hipError_t FDT_CAT2(fdt_launch_mcmc_vpl, FDT_VPL) FDT_UNIT_ARGS {
   if (a->nvox <= 0) return hipSuccess;
   if (a->acqv && a->acqv_stride < 16 * FDT_VPL) return hipErrorInvalidValue;
+  // An acquisition of 16 FDT_VPL volumes leaves no padding slot: kernels without
+  // the masks.  Measured masked -> without at 48, 80, 112, 160, 224, 288, 384, 448
+  // and 512 volumes, every model and K: Gaussian 0.2 to 5% faster (288 volumes,
+  // K=3, model 2, 24,000 voxels, 250 sweeps: 11.05 -> 10.89 ms), Rician 4 to 7%
+  // (31.8 -> 30.1, model 3), two rows 1 to 9% (4.24 -> 3.93 at 2,000 voxels).  The
+  // --gradnonlin kernels keep the masks.
+  const bool full = !a->acqv && a->N == 16 * FDT_VPL;
 #if FDT_CAN_TWO
   const bool few = a->nvox <= (rician ? 4096 : 2048);
   if (!a->acqv && (few || (FDT_ONLY_TWO && !one_row_above(K, rician))))
-    return FDT_CAT2(fdt_launch_mcmc_two_vpl, FDT_VPL)(a, K, rician, s);
+    return full ? FDT_UNIT(5)(a, K, rician, s) : FDT_UNIT(2)(a, K, rician, s);
 #endif
-  return rician ? FDT_CAT2(fdt_launch_mcmc_ric_vpl, FDT_VPL)(a, K, s) : launch<false>(a, K, s);
+#if FDT_VPL <= 28
+  if (full && !rician) return FDT_UNIT(3)(a, K, rician, s);
+#endif
+#if !FDT_ONLY_TWO
+  if (full) return FDT_UNIT(4)(a, K, rician, s);
+#endif
+  return rician ? FDT_UNIT(1)(a, K, rician, s) : launch<false>(a, K, s);
 }
 #endif
+}
