@@ -16,15 +16,19 @@ __device__ inline int xcd_tile(int b, int nb) {
 }
 
 // VPL volumes per lane in ROWS rows per voxel: a tile of VPL ROWS.
-// Waves per SIMD: two where the state allows it.  Two fibres of model 1 at 5
-// volumes per lane sit at the 128 registers of four waves, and are held to them
-// (60,000 voxels, 250 sweeps: 4.99 ms at 129 registers, 4.63 at 128).
-template <int K, int VPL, int MODEL, bool RIC, bool GN, int ROWS>
-constexpr int WAVES = ROWS == 1 && VPL <= 5 && K == 2 && MODEL == 1 && !RIC && !GN ? 4
-                      : VPL <= 18 || (K == 1 && !RIC && !GN)          ? 2
-                                                                      : 1;
+// Waves per SIMD: two where the state allows it, and above that as many as a
+// kernel's registers let in (four up to 128 of them, three up to 168): from 33 to
+// 160 volumes the chains are short series of dependent operations, which other
+// waves fill.  60,000 voxels, 250 sweeps, held to two waves -> not: 33 volumes,
+// model 2, K=1, 4.45 -> 3.65 ms; 69 volumes, K=3, 10.36 -> 9.73; 100 volumes, K=3,
+// 13.4 -> 11.8 (Rician 30.6 -> 25.8, --gradnonlin 14.5 -> 13.6); 145 volumes, K=3,
+// 17.5 -> 15.6.  Nothing changes above 168 registers: Rician chains and
+// zeppelins of three fibres at 145 volumes, and all above 160 volumes but model 2
+// with one fibre (200 volumes: 11.3 -> 9.6).
+template <int K, int VPL, bool RIC, bool GN>
+constexpr int MIN_WAVES = VPL <= 18 || (K == 1 && !RIC && !GN) ? 2 : 1;
 template <int K, int VPL, int MODEL, bool RIC, bool GN, bool FULL, int ROWS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES<K, VPL, MODEL, RIC, GN, ROWS>, WAVES<K, VPL, MODEL, RIC, GN, ROWS> > 2 ? 4 : 2))) void mcmc_kernel(McmcArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MIN_WAVES<K, VPL, RIC, GN>, 4))) void mcmc_kernel(McmcArgs a) {
   constexpr bool SMALL = Chain<K, VPL, MODEL, RIC, GN, FULL, ROWS>::SMALL;  // state in registers
   constexpr int TILE = VPL * ROWS;
   __shared__ float4 sacq[16 * TILE];
