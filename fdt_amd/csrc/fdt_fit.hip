@@ -1223,6 +1223,22 @@ FDT_DEV void store_result(const LmArgs& a, int vox, TC (&p)[NP], int total, int 
   if (a.iters && rl == 0) a.iters[vox] = (a.iters_add ? a.iters[vox] : 0) + total;
 }
 
+// Rows in step: rows whose last trip succeeded need new normal equations, the
+// others only another trial step, and a wave pays for the normal equations
+// whenever one row needs them.  Successes and failures mostly alternate, so a
+// row that needs them waits until a second one does (or no other has a trial to
+// make), and the rows fall into step: per trip of a voxel 2,264 instead of 2,676
+// instruction slots (a replay of the sequences of 480 multi-shell voxels; 2,252
+// for three rows, 2,420 for four).  Free rows -> in step: 60,000 voxels of 288
+// volumes, model 2, K=3, 80.9 -> 73.1 ms, with FP64 normal equations (--f0)
+// 20,000 voxels 94.2 -> 72.4, K=1 31.2 -> 25.6.  Where the normal equations are
+// small beside the FP64 cost of a trial, the waiting is not paid back:
+// PVM_single with two fibres (69 volumes 10.96 -> 11.27 ms for 120,000 voxels,
+// 288 volumes 15.36 -> 15.52; with three 24.6 -> 22.2 for 60,000) and with one,
+// PVM_single_c with one (69 volumes 3.29 -> 3.41; with two 11.59 -> 11.09).
+template <class T, int KIND, int K>
+constexpr bool IN_STEP = std::is_same<T, double>::value || KIND >= KIND_MULTI || K > (KIND == KIND_SINGLE_C ? 1 : 2);
+
 // GN: --gradnonlin, every voxel reads its own corrected acquisition from
 // a.acqv instead of the workgroup's table in LDS.
 template <class T, class TC, int KIND, int K, bool F0, bool GN>
@@ -1281,15 +1297,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_sam
       S.template begin<false>(R, mc0);
       fresh = false;
     }
-    // Rows whose last trip succeeded need new normal equations, the others only
-    // another trial step; a wave pays for the normal equations whenever one row
-    // does.  Successes and failures mostly alternate, so a row that needs them
-    // waits until a second one does (or no other has a trial to make), and the
-    // rows fall into step: per trip of a voxel 2,264 instead of 2,676
-    // instruction slots (a replay of the sequences of 480 multi-shell voxels;
-    // 2,252 for three rows, 2,420 for four).
-    const uint64_t need = __builtin_amdgcn_ballot_w64(S.success), all = __builtin_amdgcn_ballot_w64(true);
-    if (S.success && need != all && __builtin_popcountll(need) < 32) continue;
+    if constexpr (IN_STEP<T, KIND, K>) {
+      const uint64_t need = __builtin_amdgcn_ballot_w64(S.success), all = __builtin_amdgcn_ballot_w64(true);
+      if (S.success && need != all && __builtin_popcountll(need) < 32) continue;
+    }
     if (S.template step<false>(R, m0, mc0)) {
       store_result<TC, KIND, K, F0>(a, vox, S.p, S.total, rl);
       fresh = true;
