@@ -6,7 +6,8 @@
 //
 // GEMM: C[M x N] = A[M x K] . B[K x N] in v_mfma_f32_16x16x32_bf16 (FP32
 // accumulation).  Each operand is stored with k contiguous or with m (n)
-// contiguous, so X.W, dZ.W^T and X^T.dZ are one kernel.
+// contiguous, so X.W, dZ.W^T and X^T.dZ are one kernel (a transposed A with a
+// k-contiguous B is no product of the network and refused).
 #include "fdt_device.h"
 #include "fdt_mlp.h"
 
@@ -15,7 +16,6 @@ namespace fdt {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-FDT_DEV float bf2f(uint16_t h) { return __builtin_bit_cast(float, (uint32_t)h << 16); }
 // round to nearest even (finite inputs)
 FDT_DEV uint16_t f2bf(float x) {
   uint32_t u = __builtin_bit_cast(uint32_t, x);
@@ -346,28 +346,31 @@ __global__ void sg_fallback_kernel(SgFallbackArgs a) {
 }  // namespace fdt
 
 namespace {
-template <int TM, int TN>
+template <int TM, int TN, bool AK, bool BK>
 hipError_t launch_tile(const fdt::GemmArgs* g, hipStream_t s) {
   const int rows = g->M + (g->a.ones ? 1 : 0);
   const dim3 grid((unsigned)(((rows + TM - 1) / TM) * ((g->N + TN - 1) / TN))), block(256);
-  if (g->a.kc && g->b.kc) hipLaunchKernelGGL((fdt::gemm_bf16_kernel<TM, TN, true, true>), grid, block, 0, s, *g);
-  else if (g->a.kc) hipLaunchKernelGGL((fdt::gemm_bf16_kernel<TM, TN, true, false>), grid, block, 0, s, *g);
-  else if (!g->b.kc) hipLaunchKernelGGL((fdt::gemm_bf16_kernel<TM, TN, false, false>), grid, block, 0, s, *g);
-  else return hipErrorInvalidValue;
+  hipLaunchKernelGGL((fdt::gemm_bf16_kernel<TM, TN, AK, BK>), grid, block, 0, s, *g);
   return hipGetLastError();
+}
+// The largest tile that still gives each of the 256 CUs a workgroup
+template <bool BK>
+hipError_t launch_sized(const fdt::GemmArgs* g, hipStream_t s) {
+  auto tiles = [&](int tm, int tn) { return (long)((g->M + tm - 1) / tm) * ((g->N + tn - 1) / tn); };
+  if constexpr (!BK)  // outputs of at most 32 columns do not fill wider tiles
+    if (g->N <= 32) return tiles(128, 32) >= 256 ? launch_tile<128, 32, true, BK>(g, s) : launch_tile<32, 32, true, BK>(g, s);
+  if (tiles(128, 128) >= 256) return launch_tile<128, 128, true, BK>(g, s);
+  if (tiles(64, 64) >= 256) return launch_tile<64, 64, true, BK>(g, s);
+  return launch_tile<32, 32, true, BK>(g, s);
 }
 }  // namespace
 
-// The largest tile that still gives each of the 256 CUs a workgroup; outputs
-// of at most 32 columns do not fill wider tiles
+// Weight gradients (A with m contiguous) have at most 513 x 512 outputs, so that
+// no tile but the smallest comes near a workgroup per CU: they have that one only.
 extern "C" hipError_t fdt_launch_gemm_bf16(const fdt::GemmArgs* g, hipStream_t s) {
   if (g->M <= 0 || g->N <= 0) return hipSuccess;
-  const int rows = g->M + (g->a.ones ? 1 : 0);
-  auto tiles = [&](int tm, int tn) { return (long)((rows + tm - 1) / tm) * ((g->N + tn - 1) / tn); };
-  if (g->N <= 32) return tiles(128, 32) >= 256 ? launch_tile<128, 32>(g, s) : launch_tile<32, 32>(g, s);
-  if (tiles(128, 128) >= 256) return launch_tile<128, 128>(g, s);
-  if (tiles(64, 64) >= 256) return launch_tile<64, 64>(g, s);
-  return launch_tile<32, 32>(g, s);
+  if (g->a.kc) return g->a.ones ? hipErrorInvalidValue : g->b.kc ? launch_sized<true>(g, s) : launch_sized<false>(g, s);
+  return g->b.kc ? hipErrorInvalidValue : launch_tile<32, 32, false, false>(g, s);
 }
 
 extern "C" hipError_t fdt_launch_to_bf16(const float* x, uint16_t* y, size_t n, hipStream_t s) {
