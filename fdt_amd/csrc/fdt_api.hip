@@ -211,7 +211,7 @@ struct fdt_ctx {
   DevBuf<float> o_th, o_ph, o_f;
   DevBuf<float> m_S0, m_d, m_dstd, m_R, m_f0, m_tau, m_f, m_dyads, m_disp;
   hipEvent_t ev[6] = {};
-  int vpl_force = 0, vpl_used = 0;
+  int vpl_force = 0, vpl_used = 0, rows_used = 1;  // tile asked for; tile and rows per voxel of the last chain launch
   bool timed_fit = false, timed_mcmc = false, timed_finish = false;
   bool quiet = false;  // no timing events (launches recorded into a graph)
   uint64_t vox_offset = 0;
@@ -858,6 +858,7 @@ static int mcmc_prepare(fdt_ctx* c, uint64_t vox_offset, McmcArgs* out, mcmc_lau
     a.gdev = c->d_grad.p;
     a.nshell = 0;
   }
+  c->rows_used = mcmc_rows(a, vpl, K, o.rician);
   *out = a;
   *fn_out = fn;
   return FDT_OK;
@@ -966,6 +967,7 @@ static int spatial_async(fdt_ctx* c, uint64_t vox_offset) {
     McmcArgs b = a;
     b.list = L;
     b.nvox = n;
+    c->rows_used = mcmc_rows(b, c->vpl_used, K, false);
     HIPCHK(c, fn(&b, K, 0, c->stream));
     ss.list = L; ss.count = n;
     HIPCHK(c, fdt_launch_spatial_stats(&ss, c->stream));
@@ -1125,8 +1127,8 @@ int fdt_get_timing(fdt_ctx* c, fdt_timing* t) {
   if (c->timed_fit) HIPCHK(c, hipEventElapsedTime(&t->ms_fit, c->ev[0], c->ev[1]));
   if (c->timed_mcmc) HIPCHK(c, hipEventElapsedTime(&t->ms_mcmc, c->ev[2], c->ev[3]));
   if (c->timed_finish) HIPCHK(c, hipEventElapsedTime(&t->ms_finish, c->ev[4], c->ev[5]));
-  t->mcmc_vpl = c->vpl_used;
-  t->mcmc_lanes = 16;
+  t->mcmc_vpl = c->vpl_used / c->rows_used;
+  t->mcmc_lanes = 16 * c->rows_used;
   return FDT_OK;
 }
 

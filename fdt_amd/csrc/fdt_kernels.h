@@ -128,6 +128,32 @@ struct McmcArgs {
   const float* gdev;    // --gradnonlin: per-voxel deviation values [nvox][9]
 };
 
+// Tiles (volumes per lane of a 16-lane row) that have a kernel with one row per
+// voxel: all up to 18, and above it Gaussian chains of one fibre.
+constexpr bool mcmc_one_row(int vpl, int K, bool rician) { return vpl <= 18 || (K == 1 && !rician && vpl <= 28); }
+// Rows of 16 lanes that share a voxel in launch `a` with tile vpl: two (ms of
+// 250 sweeps, one row -> two)
+// - for launches that one-row waves would leave on half of the 1,024 SIMDs or
+//   less, 64% of whose cycles then issue: up to 2,048 voxels Gaussian, 4,096
+//   Rician.  Faster for every model and K at 113, 145, 160, 200 and 288 volumes:
+//   Gaussian by 1.2 to 1.5 from 400 to 2,048 voxels (145 volumes, K=3, model 2,
+//   1.72 -> 1.13; 288, K=1, model 3, 1.31 -> 1.08), but 3,000 voxels of 288 2.71
+//   -> 2.76; Rician by 1.5 to 1.9 up to 2,048 and 1.2 to 1.5 at 4,096 (145
+//   volumes, K=2, model 2, 3.32 -> 2.63; 288, K=3, model 3, 8.17 -> 5.48);
+// - above 288 volumes, where one row takes more than half of a SIMD's registers
+//   and leaves it one wave: 24,000 voxels of 432 volumes, model 2: K=3 24.1 ->
+//   20.4, K=2 17.2 -> 15.2, Rician model 3 K=3 74.4 -> 48.8.  Gaussian chains of
+//   one fibre fit two waves of one row up to 448 volumes and stay there (7.9
+//   against 10.3).
+// At 288 volumes and 24,000 voxels one row is faster (K=3, model 2: 11.3 against
+// 15.1; Rician model 3 30.2 against 31.2): the second row repeats every
+// proposal's sums and decision.
+inline int mcmc_rows(const McmcArgs& a, int vpl, int K, bool rician) {
+  if (a.acqv || vpl < 10) return 1;  // --gradnonlin and small tiles: one-row kernels only
+  if (!mcmc_one_row(vpl, K, rician)) return 2;
+  return a.nvox <= (rician ? 4096 : 2048) ? 2 : 1;
+}
+
 // Batched MCMC over a queue of volumes (fdt_queue.hip): work items are runs
 // of rows_per_wg consecutive voxels of one job; job j owns items
 // [first_item[j], first_item[j+1]).

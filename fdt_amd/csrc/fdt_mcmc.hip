@@ -70,27 +70,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MIN_WAVES<K
 #define FDT_CAT2_(a, b) a##b
 #define FDT_CAT2(a, b) FDT_CAT2_(a, b)
 
-// Two rows per voxel (ms of 250 sweeps, one row -> two)
-// - for launches that one-row waves would leave on half of the 1,024 SIMDs or
-//   less, 64% of whose cycles then issue: up to 2,048 voxels Gaussian (288
-//   volumes, K=3, model 2: 2.73 -> 2.13 at 2,000 voxels, but 3,000 voxels 2.71 ->
-//   2.76), 4,096 Rician (8.39 -> 4.38 at 2,000, model 3);
-// - above 288 volumes, where one row takes more than half of a SIMD's registers
-//   and leaves it one wave: 24,000 voxels of 432 volumes, model 2: K=3 24.1 ->
-//   20.4, K=2 17.2 -> 15.2, Rician model 3 K=3 74.4 -> 48.8.  Gaussian chains of
-//   one fibre fit two waves of one row up to 448 volumes and stay there (7.9
-//   against 10.3).
-// At 288 volumes and 24,000 voxels one row is faster (K=3, model 2: 11.3 against
-// 15.1; Rician model 3 30.2 against 31.2): the second row repeats every
-// proposal's sums and decision.
-#define FDT_ONLY_TWO (FDT_VPL > 18)
 #define FDT_CAN_TWO (FDT_VPL % 2 == 0 && FDT_VPL >= 10)
 
 namespace {
 constexpr bool FULL = FDT_MCMC_UNIT >= 3;
 constexpr int ROWS = FDT_MCMC_UNIT % 3 == 2 ? 2 : 1;
-// tiles above 18 that keep a one-row kernel
-constexpr bool one_row_above(int K, bool rician) { return K == 1 && !rician && FDT_VPL <= 28; }
 template <int K, int MODEL, bool RIC>
 hipError_t launch_model(const fdt::McmcArgs* a, hipStream_t s) {
   const dim3 grid((a->nvox + 16 / ROWS - 1) / (16 / ROWS)), block(256);
@@ -100,7 +84,7 @@ hipError_t launch_model(const fdt::McmcArgs* a, hipStream_t s) {
       return hipGetLastError();
     }
   }
-  if constexpr (ROWS == 2 || !FDT_ONLY_TWO || one_row_above(K, RIC)) {
+  if constexpr (ROWS == 2 || fdt::mcmc_one_row(FDT_VPL, K, RIC)) {
     hipLaunchKernelGGL((fdt::mcmc_kernel<K, FDT_VPL / ROWS, MODEL, RIC, false, FULL, ROWS>), grid, block, 0, s, *a);
     return hipGetLastError();
   }
@@ -152,14 +136,13 @@ hipError_t FDT_CAT2(fdt_launch_mcmc_vpl, FDT_VPL) FDT_UNIT_ARGS {
   // --gradnonlin kernels keep the masks.
   const bool full = !a->acqv && a->N == 16 * FDT_VPL;
 #if FDT_CAN_TWO
-  const bool few = a->nvox <= (rician ? 4096 : 2048);
-  if (!a->acqv && (few || (FDT_ONLY_TWO && !one_row_above(K, rician))))
+  if (fdt::mcmc_rows(*a, FDT_VPL, K, rician) == 2)
     return full ? FDT_UNIT(5)(a, K, rician, s) : FDT_UNIT(2)(a, K, rician, s);
 #endif
 #if FDT_VPL <= 28
   if (full && !rician) return FDT_UNIT(3)(a, K, rician, s);
 #endif
-#if !FDT_ONLY_TWO
+#if FDT_VPL <= 18
   if (full) return FDT_UNIT(4)(a, K, rician, s);
 #endif
   return rician ? FDT_UNIT(1)(a, K, rician, s) : launch<false>(a, K, s);

@@ -107,9 +107,8 @@ typedef struct fdt_timing {
   float ms_fit;     /* device time of the LM kernels of the last fdt_fit */
   float ms_mcmc;    /* device time of the MCMC kernel of the last fdt_mcmc */
   float ms_finish;  /* device time of the finish kernel of the last fdt_finish */
-  int mcmc_vpl;     /* tile of the MCMC kernel: volumes per lane of a 16-lane row (small or
-                       long launches share a tile between two rows) */
-  int mcmc_lanes;   /* lanes per row */
+  int mcmc_vpl;     /* volumes per lane chosen for the MCMC kernel */
+  int mcmc_lanes;   /* lanes per voxel: 16, or 32 where two rows share a voxel */
 } fdt_timing;
 
 typedef struct fdt_ctx fdt_ctx;

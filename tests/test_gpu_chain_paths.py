@@ -71,3 +71,26 @@ def test_filled_tiles_match_the_next_larger_one(fdt, n, larger, model, K, opts, 
     opts = dict(opts, nfibres=K, model=model)
     args = (fdt, acq, repeat(data, nvox), repeat(p, nvox), repeat(tau, nvox))
     assert_same(run(*args, **opts), run(*args, tile=larger, **opts), nvox, f"N={n} model {model} K={K} {opts}")
+
+
+@pytest.mark.parametrize("n,nvox,K,rician,lanes,vpl", [
+    (69, 100, 2, 0, 16, 5), (112, 100, 1, 1, 16, 7), (113, 2048, 2, 0, 32, 5), (160, 2049, 2, 0, 16, 10),
+    (200, 4096, 1, 1, 32, 7), (200, 4097, 1, 1, 16, 14), (288, 2049, 3, 0, 16, 18), (289, 3000, 2, 0, 32, 12),
+    (289, 3000, 1, 0, 16, 24), (448, 5000, 1, 1, 32, 14), (512, 3000, 1, 0, 32, 16)])
+def test_timing_reports_the_lanes_of_a_voxel(fdt, n, nvox, K, rician, lanes, vpl):
+    """fdt_timing: volumes per lane and lanes per voxel, of which their product holds the acquisition"""
+    acq, data, t = volume(n, 24, 1, b0=4)
+    x = fdt.Xfibres(nfibres=K, model=1, rician=rician, nburn=0, njumps=2, sampleevery=1)
+    try:
+        x.set_acquisition(*acq)
+        x.load_data(repeat(data, nvox))
+        x.set_params(repeat(starts(t, 1, K), nvox), repeat(t["tau"].astype(np.float32), nvox))
+        x.mcmc(0)
+        tm = x.timing()
+        assert (tm["lanes"], tm["vpl"]) == (lanes, vpl)
+        x.set_mcmc_tile(32)
+        x.mcmc(0)
+        tm = x.timing()
+        assert tm["lanes"] * tm["vpl"] == 512
+    finally:
+        x.close()
