@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <random>
 #include <cmath>
 #include <cstdarg>
@@ -211,6 +212,7 @@ struct fdt_ctx {
   DevBuf<float> o_th, o_ph, o_f;
   DevBuf<float> m_S0, m_d, m_dstd, m_R, m_f0, m_tau, m_f, m_dyads, m_disp;
   hipEvent_t ev[6] = {};
+  int fits_beside = 0, chains_beside = 0;  // in a batch: see LmArgs and McmcArgs
   int vpl_force = 0, vpl_used = 0, rows_used = 1;  // tile asked for; tile and rows per voxel of the last chain launch
   bool timed_fit = false, timed_mcmc = false, timed_finish = false;
   bool quiet = false;  // no timing events (launches recorded into a graph)
@@ -504,6 +506,7 @@ static LmArgs base_lm_args(fdt_ctx* c) {
   a.shell = c->d_shell.p;
   a.shell_b = c->d_shell_b.p;
   a.nshell = c->gn ? 0 : c->nshell;
+  a.beside = c->fits_beside;
   return a;
 }
 
@@ -858,6 +861,7 @@ static int mcmc_prepare(fdt_ctx* c, uint64_t vox_offset, McmcArgs* out, mcmc_lau
     a.gdev = c->d_grad.p;
     a.nshell = 0;
   }
+  a.beside = c->chains_beside;
   c->rows_used = mcmc_rows(a, vpl, K, o.rician);
   *out = a;
   *fn_out = fn;
@@ -1210,8 +1214,24 @@ static int queue_launch_chains(fdt_queue* q, const QueueJob* d_jobs, int njobs, 
   return FDT_OK;
 }
 
+// Voxels of the batch whose fits, and whose own chain launches, run at the same time: all, or the share of four volumes
+// of more (a process has four hardware queues)
+static void queue_count_beside(fdt_queue* q) {
+  long fits = 0, chains = 0, own = 0;
+  for (fdt_ctx* c : q->jobs) {
+    fits += c->nvox;
+    if (!in_queue_kernel(c)) { chains += c->nvox; ++own; }
+  }
+  auto at_once = [](long vox, long volumes) { return (int)std::min(volumes > 4 ? vox * 4 / volumes : vox, (long)INT_MAX); };
+  for (fdt_ctx* c : q->jobs) {
+    c->fits_beside = at_once(fits, (long)q->jobs.size());
+    c->chains_beside = at_once(chains, own);
+  }
+}
+
 // issue the whole batch on the queue stream (upload: also rebuild and copy the job table)
 static int queue_issue(fdt_queue* q, bool upload) {
+  queue_count_beside(q);
   QHIP(q, hipEventRecord(q->ev_fork, q->stream));
   for (fdt_ctx* c : q->jobs) {
     QHIP(q, hipStreamWaitEvent(c->stream, q->ev_fork, 0));

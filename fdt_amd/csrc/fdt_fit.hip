@@ -1313,10 +1313,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_sam
 // leaves most of the chip idle while the longest voxels finish: the learned
 // start's fallback, small volumes, parts.  A trip at 288 volumes and K=3 takes
 // 0.4 of the one-row kernel's time and 1.7 times its lanes' work.  Measured,
-// one-row kernel -> this one, both stages at 288 volumes, K=3: 200 voxels 15.6
-// -> 8.3 ms, 4,000 19.7 -> 14.9, 6,000 25.2 -> 18.7, 8,000 25.8 -> 22.2, 12,000
-// 28.3 either way.  Moving only the last voxels of a larger launch over here
-// did not pay (20,011 voxels: 45.1 instead of 40.0 ms).
+// one-row kernel -> this one, both stages, ms: 288 volumes, K=3, 500 voxels 21.5
+// -> 8.4, 4,000 25.0 -> 14.8, 6,000 24.8 -> 18.7, 8,000 25.5 -> 21.9, 12,000 28.8 ->
+// 28.7; 69 volumes, model 1, K=2, 2,000 voxels 3.6 -> 2.2, 8,000 3.9 -> 3.2.  FP64
+// (--f0, the refit's lists in this kernel either way): 2,000 voxels of 145 volumes
+// and K=2 12.4 -> 9.5; 3,000 voxels of 145 volumes 12.8 -> 11.1, of 288, K=3, 22.7
+// -> 22.6, but of 69, K=3, 19.2 -> 23.7; 4,000 12.6 -> 13.7, 33.6 -> 35.6, 20.7 ->
+// 28.5.  Moving only the last voxels of a larger launch over here did not pay
+// (20,011 voxels: 45.1 instead of 40.0 ms).
+// The volumes of a batch run at once, and a row per voxel is the better one when
+// together they fill the chip: four volumes of 33, 69, 145 and 288, fits and
+// chains, row and wave: 3,000 voxels each 52.4 and 47.4, 5,000 64.6 and 63.7, 6,000
+// 72.5 and 75.3 (the first run of a new batch 97 and 90), 7,000 85.7 and 91.4, 8,000
+// 88.6 and 96.4; two of 8,000 voxels of 145 volumes, fits, 17.2 and 15.0, three 18.6
+// and 19.6, six of 5,000 29.5 and 26.7 (four hardware queues run four of them), of
+// 8,000 33.2 and 37.5.  FP64 fits stay here up to 2,048 voxels in a batch too: four
+// of 2,000 voxels 21.0 and 24.3 at 69 volumes, K=2, but 61.4 and 55.4 at 288, K=3.
 template <class T, class TC, int KIND, int K, bool F0, bool GN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_same<T, TC>::value && std::is_same<T, double>::value ? 1 : 2, 2))) void lm_wave_kernel(LmArgs a) {
   extern __shared__ float4 lds4[];
@@ -1550,8 +1562,10 @@ hipError_t launch_lm(const fdt::LmArgs* a, hipStream_t s) {
   fdt::LmArgs b = *a;
   if (a->lm) {
     if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&wper_cu, wkern, 256, wlds)) != hipSuccess) return e;
-    // four voxels per resident wave, two where only one wave fits a SIMD (FP64)
+    // four voxels per resident wave, two where only one wave fits a SIMD (FP64); none where the batch around this
+    // launch has more than twelve (a refit list is a small part of its volume)
     b.wave_max = (wper_cu > 1 ? 16 * wper_cu : 8) * cus;
+    if (!a->count && wper_cu > 1 && a->beside > 48 * wper_cu * cus) b.wave_max = 0;
   }
   if (!a->lm || a->nvox > b.wave_max) {
     const long want = ((long)a->nvox + 3) / 4, cap = (long)std::max(per_cu, 1) * cus;

@@ -41,6 +41,7 @@ struct LmArgs {
   const int* shell;     // [N] b-shell index of each volume, or null
   const float* shell_b; // [16] b value of each shell
   int nshell;           // number of shells (0: none; ignored with acqv)
+  int beside;           // voxels whose fits run at the same time, these among them (a batch; 0: these alone)
   int wave_max;         // launches of at most so many voxels run in lm_wave_kernel alone (set by the launcher)
 };
 
@@ -126,6 +127,7 @@ struct McmcArgs {
   const float4* acqv;   // --gradnonlin: per-voxel acquisitions [nvox][acqv_stride >= Npad], or null
   int acqv_stride;
   const float* gdev;    // --gradnonlin: per-voxel deviation values [nvox][9]
+  int beside;           // voxels whose chain launches run at the same time, these among them (a batch; 0: these alone)
 };
 
 // Tiles (volumes per lane of a 16-lane row) that have a kernel with one row per
@@ -147,11 +149,19 @@ constexpr bool mcmc_one_row(int vpl, int K, bool rician) { return vpl <= 18 || (
 //   against 10.3).
 // At 288 volumes and 24,000 voxels one row is faster (K=3, model 2: 11.3 against
 // 15.1; Rician model 3 30.2 against 31.2): the second row repeats every
-// proposal's sums and decision.
+// proposal's sums and decision.  So it is, at once, for the Rician volumes of a
+// batch together (ms of 1,000 sweeps and the fits): four of 1,000 voxels 25.3 ->
+// 18.3 (145 volumes, K=2, model 2), two of 3,000 26.4 -> 26.5 (200 volumes 34.0 ->
+// 32.6), four of 2,000 27.9 -> 29.5, four of 4,000 48.6 -> 52.7.  Three fibres in
+// tiles from 14 are the exception (200 volumes, four of 2,000 75.7 -> 54.6, of
+// 4,000 111.6 -> 100.6; 288, model 3, 86.9 -> 58.4 and 123.8 -> 106.8): a CU takes
+// two of their workgroups, and those that find it taken by another volume's fits
+// wait for whole chains.
 inline int mcmc_rows(const McmcArgs& a, int vpl, int K, bool rician) {
   if (a.acqv || vpl < 10) return 1;  // --gradnonlin and small tiles: one-row kernels only
   if (!mcmc_one_row(vpl, K, rician)) return 2;
-  return a.nvox <= (rician ? 4096 : 2048) ? 2 : 1;
+  if (a.nvox > (rician ? 4096 : 2048)) return 1;
+  return a.beside <= 6144 || (K == 3 && vpl >= 14) ? 2 : 1;
 }
 
 // Batched MCMC over a queue of volumes (fdt_queue.hip): work items are runs
