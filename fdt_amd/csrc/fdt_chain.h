@@ -21,8 +21,9 @@
 // per-volume changes for its acceptance took 5,107 VALU instructions per wave
 // and sweep to 4,154, and one kernel per model (128 KB of code to 54, no
 // spilled vector registers) let the launch follow: 1,247 to 1,013 ms.  Masks
-// compiled out at 288 volumes, the draws' products from one instruction and no
-// question about a slot or a sweep number inside a sweep: 973 ms.
+// compiled out where the acquisition fills the tile (here 288 volumes), the
+// draws' products from one instruction and no question about a slot or a sweep
+// number inside a sweep: 973 ms.
 // A proposal evaluates only what it changes; its likelihood change is
 // summed over the row with DPP adds.  For Gaussian noise a move of every
 // residual by -c*q gives the change of the sum of squares c*(c*sum q^2 -

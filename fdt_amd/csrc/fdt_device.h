@@ -64,8 +64,9 @@ FDT_DEV float row_bcast(float v) {
 // total in all its lanes; the four row totals are read from lanes 0, 16, 32
 // and 48 with v_readlane and combined in a fixed order, so the result is
 // wave-uniform.  (The gfx950 permlane16/32 swaps would keep this on the VALU,
-// but ROCm 7.2 clang folds the two results of a swap whose operands are the
-// same value into one, so they are not used.)
+// but ROCm 7.2 clang gives the first of a swap's two results for the second one
+// too; the chains with two rows per voxel use one swap, and its first result
+// only.)
 FDT_DEV float rl(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
@@ -176,7 +177,8 @@ FDT_DEV u4 philox4x32_10(u4 c, uint32_t k0, uint32_t k1) {
 }
 // sqrtf of zero or of a number far from the ends of its range: the hardware's
 // root, within one ulp, moved to the neighbour on whose side of the midpoint x
-// lies.  sqrtf also scales tiny arguments and tests for infinities, seven
+// lies (Tuckerman's test, as in Markstein, IBM J. Res. Dev. 34, 1990: the root is
+// s where s (s - ulp) < x <= s (s + ulp)).  sqrtf also scales tiny arguments and tests for infinities, seven
 // instructions more; -2 log u is 0 or in [1.1e-7, 33.3].
 FDT_DEV float sqrt_nearest(float x) {
   const float s = __builtin_amdgcn_sqrtf(x);

@@ -5,10 +5,11 @@
 // consecutive voxels of one volume, one per 16-lane row) from a device
 // counter, stages that volume's acquisition in LDS and runs the chains with
 // the tile of that volume (run_chain, fdt_chain.h); it takes the next item
-// when all its rows are done.  Every (K, VPL) tile with VPL <= 18 is compiled
-// in; the register budget is that of the largest (K=3, VPL=18).  Draws are
-// keyed by each volume's global voxel index, so a voxel's chain is the same
-// as in the per-volume launch with the same tile.
+// when all its rows are done.  The tiles 3, 5, 10 and 18 are compiled in for
+// every K (the register budget is that of the largest, K=3 at 18): volumes that
+// would take 7 or 14 by themselves run in 10 or 18.  Draws are keyed by each
+// volume's global voxel index and padding adds exact zeros to every sum, so a
+// voxel's chain is the same as in the per-volume launch.
 #include "fdt_chain.h"
 
 namespace fdt {

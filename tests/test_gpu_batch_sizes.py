@@ -11,7 +11,9 @@ pytestmark = pytest.mark.gpu
 # (volumes, model, K) of each volume, their voxels: fits with a row per voxel in the batch and a wave alone (more than
 # 24,576 voxels at once), Rician chains with one row in the batch and two alone (more than 6,144; three fibres keep
 # two); the others stay below the lines
+# (200 volumes with 18 of b = 0: the queue's tile of 18 against tiles of 14 alone, in one row and in two)
 @pytest.mark.parametrize("vols,nvox,opts", [
+    ([(200, 2, 3, 18), (220, 1, 2, 18)], 2301, {}), ([(200, 3, 2, 18), (112, 2, 3, 17)], 33, dict(f0=1)),
     ([(33, 1, 1), (69, 1, 2), (100, 2, 1), (48, 2, 2)], 6501, {}),
     ([(69, 2, 2), (33, 2, 1)], 2001, dict(f0=1)),
     ([(120, 2, 2), (160, 1, 1)], 3501, dict(rician=1)),
@@ -23,8 +25,8 @@ def test_batch_equals_separate_runs(fdt, vols, nvox, opts):
     q = fdt.Queue()
     try:
         given = []
-        for j, (n, model, K) in enumerate(vols):
-            acq, data, _ = volume(n, 500, model, b0=max(2, n // 16), seed=j + 1)
+        for j, (n, model, K, *b0) in enumerate(vols):
+            acq, data, _ = volume(n, 500, model, b0=b0[0] if b0 else max(2, n // 16), seed=j + 1)
             given.append((acq, repeat(data, nvox), dict(run, nfibres=K, model=model)))
             q.enqueue(*acq, given[-1][1], vox_offset=j * nvox, **given[-1][2])
         for _ in range(2):  # issued, then replayed
